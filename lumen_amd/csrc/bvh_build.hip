@@ -645,6 +645,21 @@ __global__ void k_collapse(const Task* __restrict__ in, uint32_t n_in, Task* __r
         ex[k] = e;
         nd.e[k] = (int8_t)e;
     }
+    // internal children in the order of their centres along the longest axis
+    // (the traversal's visit order): insertion sort of at most 8
+    const int axis = ex[2] > max(ex[0], ex[1]) ? 2 : (ex[1] > ex[0] ? 1 : 0);
+    for (int i = 1; i < (int)n_int; i++) {
+        const uint32_t ci = ch[i];
+        const Box bi = cb[i];
+        const float key = bi.lo[axis] + bi.hi[axis];
+        int j = i;
+        for (; j > 0 && cb[j - 1].lo[axis] + cb[j - 1].hi[axis] > key; j--) {
+            ch[j] = ch[j - 1];
+            cb[j] = cb[j - 1];
+        }
+        ch[j] = ci;
+        cb[j] = bi;
+    }
     nd.imask = 0;
     nd.child_base = child_base;
     nd.tri_base = tri_base;
@@ -901,6 +916,14 @@ lt_status bvh_build(lt_context* ctx, const lt_build_opts* opts, lt_build_stats* 
                         }
                     }
                 }
+            }
+        }
+        {
+            Node8 root;
+            BCHK(hipMemcpy(&root, bvh.nodes, sizeof(root), hipMemcpyDeviceToHost));
+            for (int k = 0; k < 3; k++) {
+                bvh.root_p[k] = root.p[k];
+                bvh.root_x[k] = std::ldexp(131072.0f, root.e[k]);
             }
         }
         bvh.built = true;

@@ -13,7 +13,9 @@
 //          12..14  e.x e.y e.z         int8 exponents
 //          15      imask               bit i: child i is an internal node; the
 //                                      internal children fill the low slots, so
-//                                      imask = 2^n_internal - 1
+//                                      imask = 2^n_internal - 1, in the order of
+//                                      their box centres along the node's longest
+//                                      axis (the first of the largest exponents)
 //          16..19  child_base          node index of the first internal child
 //          20..23  tri_base            index of the first triangle record
 //          24..31  meta[8]             internal: its slot (node child_base + slot)

@@ -13,6 +13,15 @@
 // Stack: a per-thread short stack in LDS (kLdsStack entries, stride = block
 // size so a wave's accesses are bank-conflict free), continued in a global
 // spill area (kStackTotal - kLdsStack entries per resident thread).
+//
+// What bounds it: VALU issue, at the few lanes of a wave that still traverse
+// (node and triangle fetches are served by the caches).  The node step is
+// therefore kept short: everything that depends on the ray alone (slab error
+// bounds, cull margin) is set once per ray, the children's order comes from
+// one axis of the node, and a node's hit leaves are queued as one entry
+// (against per-node bounds, a nearest-child search and an entry per leaf:
+// 2.07M bounce rays over the 1M-triangle terrain 733 -> 636 us, the 1080p Path
+// frame 3.92 -> 3.56 ms).
 #pragma once
 #include "bvh_layout.h"
 #include "context.h"
@@ -24,6 +33,8 @@ struct RayPre {
     int kx, ky, kz;
     float Sx, Sy, Sz;
     f3 inv;
+    f3 err;        // per axis: bound on the rounding of a slab distance
+    float margin;  // bound on the rounding of a watertight t
 };
 
 LT_DEV float sel(f3 v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : v.z); }
@@ -103,7 +114,30 @@ struct HitRec {
 // a = 2^e * inv and b = (p - o) * inv each carry one rounding, inv one more
 // and the fused multiply-add one, i.e. |error| < 4 eps (65535 |a| + |b|)
 // (planes are at most 65504).
-constexpr float kSlabErr = 4.76837158e-7f;
+constexpr float kSlabErr = 4.76837158e-7f;  // 2^-21
+
+// The ray's bounds over every node of the tree: with the root at p_r and its
+// planes spanning X = 65536 2^e_r (2 X = sv.root_x), every node has
+// 65535 2^e <= X and p_r <= p <= p_r + X, so F = |1/d| (|p_r - o| + 2 X) is at
+// least 65535 |a| + |b| of every node, and at least the distance along the
+// axis of every point of its planes.  Per ray instead of per node this costs
+// a looser culling (a rounding bound of the scene's size rather than the
+// node's, 1e-6 of the scene) and saves 17 of the node step's instructions.
+//   err    2^-21 F per axis: [t_near - err, t_far + err] contains a child's
+//          true slab interval;
+//   margin 2^-16 F of the dominant axis: the watertight t of a triangle
+//          carries an absolute error of a few ulp of the largest sheared z of
+//          its vertices, i.e. of the farthest t of its boxes along that axis.
+//          Children are kept if they reach [tmin - margin, tcur + margin], so
+//          a triangle whose computed t undercuts the current best by that
+//          error is still tested.
+LT_DEV void ray_bounds(const SceneView& sv, f3 o, RayPre& rp) {
+    const f3 F = {fabsf(rp.inv.x) * (fabsf(sv.root_p[0] - o.x) + sv.root_x[0]),
+                  fabsf(rp.inv.y) * (fabsf(sv.root_p[1] - o.y) + sv.root_x[1]),
+                  fabsf(rp.inv.z) * (fabsf(sv.root_p[2] - o.z) + sv.root_x[2])};
+    rp.err = kSlabErr * F;
+    rp.margin = sel(F, rp.kz) * (1.0f / 65536.0f);
+}
 
 // LDS-qualified so that stack accesses compile to ds_read / ds_write rather
 // than flat accesses through the generic address space
@@ -117,40 +151,41 @@ struct TraceStack {
         : lds((lds_u32*)lds_col), q((lds_u32*)lds_col + ltb::kLdsStack * kTraceBlock), spill(spill_area) {}
 };
 
-LT_DEV void stk_push(const TraceStack& s, uint32_t& sp, uint32_t v) {
-    if (sp < (uint32_t)ltb::kLdsStack)
-        s.lds[sp * kTraceBlock] = v;
+// entry i of the stack; a tree of at most kLdsStack + 1 levels (sv.deep_stack
+// == 0, uniform) never leaves the LDS part
+LT_DEV void stk_set(const SceneView& sv, const TraceStack& s, uint32_t i, uint32_t v) {
+    if (sv.deep_stack && i >= (uint32_t)ltb::kLdsStack)
+        s.spill[i - ltb::kLdsStack] = v;
     else
-        s.spill[sp - ltb::kLdsStack] = v;
-    sp++;
+        s.lds[i * kTraceBlock] = v;
 }
-LT_DEV uint32_t stk_pop(const TraceStack& s, uint32_t& sp) {
-    sp--;
-    return sp < (uint32_t)ltb::kLdsStack ? s.lds[sp * kTraceBlock] : s.spill[sp - ltb::kLdsStack];
-}
-LT_DEV uint32_t stk_top(const TraceStack& s, uint32_t sp) {
-    return sp - 1 < (uint32_t)ltb::kLdsStack ? s.lds[(sp - 1) * kTraceBlock] : s.spill[sp - 1 - ltb::kLdsStack];
-}
-LT_DEV void stk_set_top(const TraceStack& s, uint32_t sp, uint32_t v) {
-    if (sp - 1 < (uint32_t)ltb::kLdsStack)
-        s.lds[(sp - 1) * kTraceBlock] = v;
-    else
-        s.spill[sp - 1 - ltb::kLdsStack] = v;
+LT_DEV uint32_t stk_get(const SceneView& sv, const TraceStack& s, uint32_t i) {
+    if (sv.deep_stack && i >= (uint32_t)ltb::kLdsStack) return s.spill[i - ltb::kLdsStack];
+    return s.lds[i * kTraceBlock];
 }
 
-// a lane takes its next node while at most this many leaf entries are queued
+// a lane takes its next node while at most this many words of leaf groups are
+// queued (0: only once every triangle it has hit the box of is tested)
 #ifndef LT_NODE_PEND_MAX
 #define LT_NODE_PEND_MAX (ltb::kLeafQueue - 8)
 #endif
-// a node step queues up to 8 more entries: the queue must hold them
+// a node step queues one group (2 words) more: the queue must hold it
 static_assert(LT_NODE_PEND_MAX >= 0 && LT_NODE_PEND_MAX + 8 <= (int)ltb::kLeafQueue,
-              "LT_NODE_PEND_MAX + 8 leaf entries exceed the per-lane LDS leaf queue");
+              "LT_NODE_PEND_MAX + 8 words exceed the per-lane LDS leaf queue");
 
-// A stack entry is a group of sibling internal nodes still to visit:
-// (child_base << 8) | mask over their slots (the internal children fill the
-// low slots, child slot c is node child_base + c).  One entry per tree level
-// instead of one per child; the group's nodes are visited from the highest
-// slot down.
+// A node's internal children lie along its longest axis in slot order (the
+// builder sorts them by their centres; the axis is the one of the largest
+// exponent, the first of equals), so a ray that runs up the axis visits the
+// hit ones from the lowest slot up and one that runs down it from the highest
+// slot down: nearly front to back, without comparing their entry distances.
+//
+// A stack entry is the group of a node's hit internal children that still wait
+// after the first: seven slots at most, because the first is the lowest
+// (upward) or the highest (downward) hit one.
+//   upward:   (child_base << 8) | slots (bits 1..7) | 1; lowest bit next
+//   downward: (child_base - 1) << 8 | slots << 1 (bits 1..7); highest bit next
+// Either way bit b is node (entry >> 8) + b, and the builder caps a BVH at
+// 2^24 nodes.  One entry per tree level instead of one per child.
 constexpr uint32_t kNoNode = 0xFFFFFFFFu;
 
 // The traversal of one query as a state machine, so that a lane can take a
@@ -158,76 +193,64 @@ constexpr uint32_t kNoNode = 0xFFFFFFFFu;
 struct TraceState {
     f3 o, d;
     RayPre rp;
-    float tmin, tmax, tcur;
+    float tmin, tmax;
+    float lo, hi;  // cull limits: tmin - margin, current best t + margin
     HitRec best;
     uint32_t sp;
-    uint32_t next;  // node to visit next (the nearest hit child), or kNoNode
-    uint32_t pend;  // leaf entries queued, (first triangle << 3) | count each
+    uint32_t next;           // node to visit next, or kNoNode
+    uint32_t tri_base, tris; // leaf group being tested: bit i is triangle tri_base + i
+    uint32_t qn;             // words of further leaf groups queued in LDS
 };
 
-LT_DEV void trace_init(TraceState& s, const TraceStack& stk, f3 o, f3 d, float tmin, float tmax, bool has_nodes) {
+LT_DEV void trace_init(const SceneView& sv, TraceState& s, f3 o, f3 d, float tmin, float tmax) {
     s.o = o;
     s.d = d;
     s.tmin = tmin;
     s.tmax = tmax;
-    s.tcur = tmax;
     s.best.gid = 0xFFFFFFFFu;
     s.best.t = tmax;
     s.best.prim = s.best.inst = 0xFFFFFFFFu;
     s.best.u = s.best.v = 0.0f;
     s.rp = prep_ray(d);
+    ray_bounds(sv, o, s.rp);
+    s.lo = tmin - s.rp.margin;
+    s.hi = tmax + s.rp.margin;
     s.sp = 0;
-    s.pend = 0;
-    s.next = has_nodes ? 0u : kNoNode;
-    (void)stk;
+    s.qn = 0;
+    s.tri_base = s.tris = 0u;
+    s.next = sv.num_nodes != 0 ? 0u : kNoNode;
 }
 
-// Processes one BVH8 node (its children's boxes, then its leaf triangles,
-// then pushes the hit internal children, nearest last).  any: finishes at the
-// first hit in [tmin, tmax] (a per-lane flag; constant where trace_step's
-// template argument gives it).  Counters are only updated when COUNT.
+// Processes one BVH8 node (its children's boxes; the hit leaves' triangles are
+// queued, the hit internal children pushed) and tests one queued triangle.
+// any: finishes at the first hit in [tmin, tmax] (a per-lane flag; constant
+// where trace_step's template argument gives it).  Counters are only updated
+// when COUNT.
 template <bool COUNT>
 LT_DEV bool trace_step_dyn(const SceneView& sv, TraceState& s, const TraceStack& stk, bool any, uint32_t& n_nodes,
                            uint32_t& n_tris) {
-    const bool has_node = s.next != kNoNode || s.sp != 0;
-    if (!has_node && s.pend == 0) return true;
     const f3 o = s.o;
     const RayPre& rp = s.rp;
-    const float tmin = s.tmin, tmax = s.tmax;
-    float& tcur = s.tcur;
     HitRec& best = s.best;
-    uint32_t& sp = s.sp;
-    if (has_node && s.pend <= (uint32_t)LT_NODE_PEND_MAX) {
-        uint32_t ni = s.next;
-        if (ni == kNoNode) {
-            const uint32_t e = stk_top(stk, sp);
-            const uint32_t ranks = e & 0xFFu;
-            const uint32_t r = 31u - (uint32_t)__builtin_clz(ranks);
-            const uint32_t left = ranks & ~(1u << r);
-            if (left)
-                stk_set_top(stk, sp, (e & ~0xFFu) | left);
-            else
-                sp--;
-            ni = (e >> 8) + r;
-        }
-        s.next = kNoNode;
+    if (s.next != kNoNode && (LT_NODE_PEND_MAX == 0 ? s.tris == 0u : s.qn <= (uint32_t)LT_NODE_PEND_MAX)) {
         if (COUNT) n_nodes++;
         // 32-bit byte offsets from the node array (scalar base + vector offset
         // addressing; the builder caps a BVH at 2^24 nodes)
         const char* nbase = (const char*)sv.nodes;
-        const uint32_t noff = ni * 128u;
+        const uint32_t noff = s.next * 128u;
         const float4 w0 = *(const float4*)(nbase + noff);
         const uint4 w1 = *(const uint4*)(nbase + (noff + 16u));
         // near / far planes by the ray octant: the plane vectors sit at
         // 16-byte slots 2..4 (qlo x, y, z) and 5..7 (qhi), so the octant picks
         // the load address instead of selecting between loaded words
         const bool negx = rp.inv.x < 0.0f, negy = rp.inv.y < 0.0f, negz = rp.inv.z < 0.0f;
-        const uint4 qnx = *(const uint4*)(nbase + (noff + (negx ? 80u : 32u)));
-        const uint4 qfx = *(const uint4*)(nbase + (noff + (negx ? 32u : 80u)));
-        const uint4 qny = *(const uint4*)(nbase + (noff + (negy ? 96u : 48u)));
-        const uint4 qfy = *(const uint4*)(nbase + (noff + (negy ? 48u : 96u)));
-        const uint4 qnz = *(const uint4*)(nbase + (noff + (negz ? 112u : 64u)));
-        const uint4 qfz = *(const uint4*)(nbase + (noff + (negz ? 64u : 112u)));
+        const uint32_t noff2 = noff + 48u;
+        const uint4 qnx = *(const uint4*)(nbase + ((negx ? noff2 : noff) + 32u));
+        const uint4 qfx = *(const uint4*)(nbase + ((negx ? noff : noff2) + 32u));
+        const uint4 qny = *(const uint4*)(nbase + ((negy ? noff2 : noff) + 48u));
+        const uint4 qfy = *(const uint4*)(nbase + ((negy ? noff : noff2) + 48u));
+        const uint4 qnz = *(const uint4*)(nbase + ((negz ? noff2 : noff) + 64u));
+        const uint4 qfz = *(const uint4*)(nbase + ((negz ? noff : noff2) + 64u));
         const uint32_t ew = __float_as_uint(w0.w);  // e.x, e.y, e.z, imask
         const int ex = (int)(int8_t)(ew & 0xFF), ey = (int)(int8_t)((ew >> 8) & 0xFF),
                   ez = (int)(int8_t)((ew >> 16) & 0xFF);
@@ -235,33 +258,17 @@ LT_DEV bool trace_step_dyn(const SceneView& sv, TraceState& s, const TraceStack&
         const uint32_t child_base = w1.x, tri_base = w1.y;
         const uint32_t meta_lo = w1.z, meta_hi = w1.w;
         // Slab distances of the children: t = q * a + b per axis with
-        // a = 2^e / d and b = (p - o) / d.  E bounds the rounding of that
-        // evaluation against the exact (p + q 2^e - o) / d, so
-        // [t_near - E, t_far + E] contains every child's true slab interval.
-        // 2^e * inv, exact (a power-of-two scaling), as one ldexp
+        // a = 2^e / d (exact, one ldexp) and b = (p - o) / d, widened by err
         const float ax = ldexpf(rp.inv.x, ex);
         const float ay = ldexpf(rp.inv.y, ey);
         const float az = ldexpf(rp.inv.z, ez);
-        const float bx = (w0.x - o.x) * rp.inv.x, by = (w0.y - o.y) * rp.inv.y, bz = (w0.z - o.z) * rp.inv.z;
-        const float Ex = kSlabErr * fmaf(65535.0f, fabsf(ax), fabsf(bx));
-        const float Ey = kSlabErr * fmaf(65535.0f, fabsf(ay), fabsf(by));
-        const float Ez = kSlabErr * fmaf(65535.0f, fabsf(az), fabsf(bz));
-        const float bnx = bx - Ex, bfx = bx + Ex, bny = by - Ey, bfy = by + Ey, bnz = bz - Ez, bfz = bz + Ez;
-        // The watertight t of a triangle carries an absolute error of a few ulp
-        // of the largest sheared z of its vertices, i.e. of the farthest t of
-        // the enclosing box along the dominant axis kz.  Children are kept if
-        // they reach [tmin - margin, tcur + margin], so a triangle whose computed
-        // t undercuts the current best by that error is still tested.
-        const float akz = rp.kz == 0 ? ax : (rp.kz == 1 ? ay : az);
-        const float bkz = rp.kz == 0 ? bx : (rp.kz == 1 ? by : bz);
-        const float far_kz = fmaxf(fabsf(bkz), fabsf(fmaf(65535.0f, akz, bkz)));
-        const float margin = far_kz * (1.0f / 65536.0f);
-        const float lo_lim = tmin - margin;
-        const float hi_lim = tcur + margin;
-        uint32_t hm = 0;
-        float tn_c[8];
+        const float dx = w0.x - o.x, dy = w0.y - o.y, dz = w0.z - o.z;
+        const float bnx = fmaf(dx, rp.inv.x, -rp.err.x), bfx = fmaf(dx, rp.inv.x, rp.err.x);
+        const float bny = fmaf(dy, rp.inv.y, -rp.err.y), bfy = fmaf(dy, rp.inv.y, rp.err.y);
+        const float bnz = fmaf(dz, rp.inv.z, -rp.err.z), bfz = fmaf(dz, rp.inv.z, rp.err.z);
+        uint32_t miss = 0;  // the sign of t1 - t0 shifts in, child 7 first
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
+        for (int c = 7; c >= 0; c--) {
             const int sh = (c & 1) * 16;
             const int wd = c >> 1;
             auto lane16 = [&](const uint4& q) {  // the fp16 plane; the fma below takes it as is
@@ -270,91 +277,90 @@ LT_DEV bool trace_step_dyn(const SceneView& sv, TraceState& s, const TraceStack&
             };
             float t0 = fmaxf(fmaxf(fmaf(lane16(qnx), ax, bnx), fmaf(lane16(qny), ay, bny)), fmaf(lane16(qnz), az, bnz));
             float t1 = fminf(fminf(fmaf(lane16(qfx), ax, bfx), fmaf(lane16(qfy), ay, bfy)), fmaf(lane16(qfz), az, bfz));
-            t0 = fmaxf(t0, lo_lim);
-            t1 = fminf(t1, hi_lim);
-            tn_c[c] = t0;
-            hm |= (t0 <= t1 ? 1u : 0u) << c;
+            t0 = fmaxf(t0, s.lo);
+            t1 = fminf(t1, s.hi);
+            // (miss << 1) | sign(t1 - t0); equal distances give +0, a NaN (both
+            // infinite) the default positive one: a hit
+            miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(t1 - t0), 31);
         }
-        const uint32_t hit_int = hm & imask;
+        const uint32_t hit_int = imask & ~miss;
         // hit slots that are not internal: leaves, and (rarely, within the
-        // rounding margin) empty slots, whose count of 0 tests nothing
-        uint32_t hit_leaf = hm & ~imask;
-        // the hit leaves join the lane's queue; their triangles are tested
-        // below, a few lanes' worth at a time
-        while (hit_leaf) {
-            const int c = __builtin_ctz(hit_leaf);
-            hit_leaf &= hit_leaf - 1;
-            const uint32_t meta = ((c < 4 ? meta_lo : meta_hi) >> ((c & 3) * 8)) & 0xFF;
-            if (meta & 7u) {
-                stk.q[s.pend * kTraceBlock] = ((tri_base + (meta >> 3)) << 3) | (meta & 7u);
-                s.pend++;
+        // rounding margin) empty slots, whose count of 0 queues nothing
+        uint32_t hit_leaf = ~miss & ~imask & 0xFFu;
+        if (hit_leaf) {
+            uint32_t m = 0u;
+            do {
+                const int c = __builtin_ctz(hit_leaf);
+                hit_leaf &= hit_leaf - 1;
+                const uint32_t meta = ((c < 4 ? meta_lo : meta_hi) >> ((c & 3) * 8)) & 0xFF;
+                m |= ((1u << (meta & 7u)) - 1u) << (meta >> 3);  // offsets and counts: at most 32 triangles
+            } while (hit_leaf);
+            if (s.tris == 0u) {
+                s.tri_base = tri_base;
+                s.tris = m;
+            } else if (m) {
+                stk.q[s.qn * kTraceBlock] = tri_base;
+                stk.q[(s.qn + 1u) * kTraceBlock] = m;
+                s.qn += 2u;
             }
         }
+        // the longest axis' direction decides the order of the children
+        const bool up = ez > max(ex, ey) ? !negz : (ey > ex ? !negy : !negx);
         if (hit_int) {
-            // nearest internal child is pushed last (popped first); it starts
-            // at the first hit child, so that it names a hit child even if no
-            // entry distance compares below +inf (an overflowed slab)
-            int nearest = __builtin_ctz(hit_int);
-            // an occlusion query takes its children in slot order: any hit
-            // ends it, and without the nearest-first choice it also visits
-            // fewer nodes (a host replay of the BVH8s: 9.3 -> 9.0 nodes per
-            // shadow ray on a terrain, 9.5 -> 8.4 on the caustics scene)
-            if (!any) {
-                float tbest = INFINITY;
-#pragma unroll
-                for (int c = 0; c < 8; c++)
-                    if (((hit_int >> c) & 1u) && tn_c[c] < tbest) {
-                        tbest = tn_c[c];
-                        nearest = c;
-                    }
+            const uint32_t first = up ? (uint32_t)__builtin_ctz(hit_int) : 31u - (uint32_t)__builtin_clz(hit_int);
+            const uint32_t rest = hit_int ^ (1u << first);
+            s.next = child_base + first;
+            if (rest) {
+                stk_set(sv, stk, s.sp, up ? ((child_base << 8) | rest | 1u) : (((child_base - 1u) << 8) | (rest << 1)));
+                s.sp++;
             }
-            // the nearest is visited next; the others wait as one group and
-            // are visited from the highest slot down (internal children fill
-            // the low slots: child c is node child_base + c)
-            const uint32_t rest = hit_int & ~(1u << nearest);
-            if (rest) stk_push(stk, sp, (child_base << 8) | rest);
-            s.next = child_base + (uint32_t)nearest;
+        } else if (s.sp != 0u) {
+            const uint32_t e = stk_get(sv, stk, s.sp - 1u);
+            const uint32_t slots = e & 0xFEu;
+            const uint32_t r =
+                (e & 1u) ? (uint32_t)__builtin_ctz(slots) : 31u - (uint32_t)__builtin_clz(slots);
+            const uint32_t left = e ^ (1u << r);
+            if (left & 0xFEu)
+                stk_set(sv, stk, s.sp - 1u, left);
+            else
+                s.sp--;
+            s.next = (e >> 8) + r;
+        } else {
+            s.next = kNoNode;
         }
     }
     // One queued triangle per lane and step: a node step and a triangle test
     // share the step instead of the wave looping over the most leaf hits of
     // any lane.  The other queued triangles wait for the next steps, which
-    // only delays the shrinking of tcur (culling stays conservative); an
-    // any-hit query ends at its first hit.
-    if (s.pend != 0u) {
-        const uint32_t e = stk.q[(s.pend - 1) * kTraceBlock];
-        const uint32_t cnt = e & 7u;
-        if (cnt == 1u)
-            s.pend--;
-        else
-            stk.q[(s.pend - 1) * kTraceBlock] = e - 1u;
-        const float4* tp = (const float4*)(sv.tris + (e >> 3) + cnt - 1u);
-        const float4 a = tp[0], b = tp[1], cc = tp[2];
+    // only delays the shrinking of the cull limit (culling stays
+    // conservative); an any-hit query ends at its first hit.
+    if (s.tris != 0u) {
+        const uint32_t b = (uint32_t)__builtin_ctz(s.tris);
+        s.tris &= s.tris - 1u;
+        const float4* tp = (const float4*)(sv.tris + (size_t)(s.tri_base + b));
+        const float4 a = tp[0], bb = tp[1], cc = tp[2];
         if (COUNT) n_tris++;
+        if (s.tris == 0u && s.qn != 0u) {
+            s.qn -= 2u;
+            s.tri_base = stk.q[s.qn * kTraceBlock];
+            s.tris = stk.q[(s.qn + 1u) * kTraceBlock];
+        }
         float t, u, v;
-        if (isect_tri(mk3(a.x, a.y, a.z), mk3(a.w, b.x, b.y), mk3(b.z, b.w, cc.x), o, rp, tmin, tmax, t, u, v)) {
+        if (isect_tri(mk3(a.x, a.y, a.z), mk3(a.w, bb.x, bb.y), mk3(bb.z, bb.w, cc.x), o, rp, s.tmin, s.tmax, t, u, v)) {
             const uint32_t gid = __float_as_uint(cc.y);
-            if (any) {
+            if (any || t < best.t || (t == best.t && gid < best.gid)) {
                 best.t = t;
                 best.u = u;
                 best.v = v;
                 best.gid = gid;
                 best.prim = __float_as_uint(cc.z);
                 best.inst = __float_as_uint(cc.w);
-                return true;
-            }
-            if (t < best.t || (t == best.t && gid < best.gid)) {
-                best.t = t;
-                best.u = u;
-                best.v = v;
-                best.gid = gid;
-                best.prim = __float_as_uint(cc.z);
-                best.inst = __float_as_uint(cc.w);
-                tcur = t;
+                s.hi = t + rp.margin;
+                if (any) return true;
             }
         }
     }
-    return s.next == kNoNode && sp == 0 && s.pend == 0u;
+    return s.next == kNoNode && s.tris == 0u;
 }
 
 template <bool ANY, bool COUNT>
@@ -392,7 +398,7 @@ LT_DEV void trace_stream(const SceneView& sv, const TraceStack& stk, uint32_t n_
                         f3 o, d;
                         float tmin, tmax;
                         tag = load(mine, o, d, tmin, tmax);
-                        trace_init(s, stk, o, d, tmin, tmax, sv.num_nodes != 0);
+                        trace_init(sv, s, o, d, tmin, tmax);
                         has = true;
                     }
                 }
@@ -435,7 +441,7 @@ LT_DEV void trace_stream_mixed(const SceneView& sv, const TraceStack& stk, uint3
                         f3 o, d;
                         float tmin, tmax;
                         tag = load(mine, o, d, tmin, tmax, any);
-                        trace_init(s, stk, o, d, tmin, tmax, sv.num_nodes != 0);
+                        trace_init(sv, s, o, d, tmin, tmax);
                         has = true;
                     }
                 }
@@ -457,7 +463,7 @@ template <bool ANY, bool COUNT>
 LT_DEV bool trace_bvh(const SceneView& sv, f3 o, f3 d, float tmin, float tmax, HitRec& best, const TraceStack& stk,
                       uint32_t& n_nodes, uint32_t& n_tris) {
     TraceState s;
-    trace_init(s, stk, o, d, tmin, tmax, sv.num_nodes != 0);
+    trace_init(sv, s, o, d, tmin, tmax);
     while (!trace_step<ANY, COUNT>(sv, s, stk, n_nodes, n_tris)) {
     }
     best = s.best;

@@ -1,13 +1,14 @@
 // oracle_bvh8.cpp — host traversal of the device-built BVH8 (TEST INFRASTRUCTURE).
 //
 // Walks the exported 128-byte nodes with the same child decode, slab test and
-// child order as the device kernel (nearest child first for closest-hit
-// queries, slot order for occlusion queries), testing a node's leaf
-// triangles at once (the device queues them and tests one per step, so its
-// closest-hit bound shrinks later): its per-ray node and triangle counts are
-// the device's lower bound, and its hits must equal the device's and brute
+// child order as the device kernel (the internal children along the node's
+// longest axis, up or down it with the ray), testing a node's leaf triangles
+// at once (the device queues them and tests one per step, so its closest-hit
+// bound shrinks later): its per-ray node and triangle counts are the device's
+// lower bound, and its hits must equal the device's and brute
 // force (oracle_trace.cpp), which isolates build defects from traversal
 // defects.
+#include <algorithm>
 #include <vector>
 
 #include "oracle.h"
@@ -58,6 +59,21 @@ extern "C" void ora_bvh8_trace(const void* nodes_v, uint32_t n_nodes, const void
         uint32_t best_gid = 0xFFFFFFFFu, best_prim = 0xFFFFFFFFu, best_inst = 0xFFFFFFFFu;
         uint64_t nn = 0, nt = 0;
         bool done = false;
+        // rounding bounds of the ray over every node of the tree (from the
+        // root): E of a slab distance per axis, 2^-21 F with
+        // F = |1/d| (|p_r - o| + 2^17 2^e_r) >= 65535 |a| + |b| of any node, and
+        // the cull margin, 2^-16 F along the dominant axis kz (the error of a
+        // triangle's watertight t)
+        float E[3] = {0, 0, 0}, margin = 0.0f;
+        if (n_nodes) {
+            const float adx = fabsf(d.x), ady = fabsf(d.y), adz = fabsf(d.z);
+            const int kz = (adx > ady) ? (adx > adz ? 0 : 2) : (ady > adz ? 1 : 2);
+            for (int k = 0; k < 3; k++) {
+                const float F = fabsf(inv[k]) * (fabsf(nodes[0].p[k] - o[k]) + ldexpf(131072.0f, nodes[0].e[k]));
+                E[k] = kSlabErr * F;
+                if (k == kz) margin = F * (1.0f / 65536.0f);
+            }
+        }
         std::vector<uint32_t> stack;
         if (n_nodes) stack.push_back(0);
         while (!stack.empty() && !done) {
@@ -65,26 +81,14 @@ extern "C" void ora_bvh8_trace(const void* nodes_v, uint32_t n_nodes, const void
             stack.pop_back();
             nn++;
             // child slab distances t = q * a + b, a = 2^e / d, b = (p - o) / d,
-            // widened by the rounding bound E = 2^-21 (65535 |a| + |b|)
-            float a[3], b[3], bn[3], bf[3];
+            // widened by the rounding bound E
+            float a[3], bn[3], bf[3];
             for (int k = 0; k < 3; k++) {
-                uint32_t bits = (uint32_t)(nd.e[k] + 127) << 23;
-                float s;
-                memcpy(&s, &bits, 4);
-                a[k] = s * inv[k];
-                b[k] = (nd.p[k] - o[k]) * inv[k];
-                float E = kSlabErr * fmaf(65535.0f, fabsf(a[k]), fabsf(b[k]));
-                bn[k] = b[k] - E;
-                bf[k] = b[k] + E;
+                a[k] = ldexpf(inv[k], nd.e[k]);
+                bn[k] = fmaf(nd.p[k] - o[k], inv[k], -E[k]);
+                bf[k] = fmaf(nd.p[k] - o[k], inv[k], E[k]);
             }
-            // cull margin: 2^-16 of the node's far t along the dominant axis kz
-            // (bounds the error of a contained triangle's watertight t)
-            float adx = fabsf(d.x), ady = fabsf(d.y), adz = fabsf(d.z);
-            int kz = (adx > ady) ? (adx > adz ? 0 : 2) : (ady > adz ? 1 : 2);
-            float far_kz = fmaxf(fabsf(b[kz]), fabsf(fmaf(65535.0f, a[kz], b[kz])));
-            float margin = far_kz * (1.0f / 65536.0f);
             uint32_t hit_int = 0, hit_leaf = 0;
-            float tn[8];
             for (int c = 0; c < 8; c++) {
                 float qn[3], qf[3];
                 for (int k = 0; k < 3; k++) {
@@ -96,8 +100,7 @@ extern "C" void ora_bvh8_trace(const void* nodes_v, uint32_t n_nodes, const void
                 float t1 = fminf(fminf(fmaf(qf[0], a[0], bf[0]), fmaf(qf[1], a[1], bf[1])), fmaf(qf[2], a[2], bf[2]));
                 t0 = fmaxf(t0, tmin - margin);
                 t1 = fminf(t1, tcur + margin);
-                bool h = t0 <= t1;  // an empty slot carries no internal bit and no count
-                tn[c] = t0;
+                bool h = !(t1 - t0 < 0.0f);  // an empty slot carries no internal bit and no count
                 bool internal = (nd.imask >> c) & 1u;
                 if (h && internal) hit_int |= 1u << c;
                 if (h && !internal && (nd.meta[c] & 7u)) hit_leaf |= 1u << c;
@@ -123,17 +126,14 @@ extern "C" void ora_bvh8_trace(const void* nodes_v, uint32_t n_nodes, const void
                 }
             }
             if (done || !hit_int) continue;
-            int nearest = __builtin_ctz(hit_int);  // occlusion queries: slot order, as the device
-            float tb = INFINITY;
-            if (!any_hit)
-                for (int c = 0; c < 8; c++)
-                    if (((hit_int >> c) & 1u) && tn[c] < tb) {
-                        tb = tn[c];
-                        nearest = c;
-                    }
-            for (int c = 0; c < 8; c++)
-                if (((hit_int >> c) & 1u) && c != nearest) stack.push_back(nd.child_base + nd.meta[c]);
-            stack.push_back(nd.child_base + nd.meta[nearest]);
+            // longest axis: the first of the largest exponents; the next child
+            // is the lowest hit slot if the ray runs up it, else the highest
+            const int axis = nd.e[2] > std::max(nd.e[0], nd.e[1]) ? 2 : (nd.e[1] > nd.e[0] ? 1 : 0);
+            const bool up = !(inv[axis] < 0.0f);
+            for (int k = 0; k < 8; k++) {
+                const int c = up ? 7 - k : k;  // pushed last, visited first
+                if ((hit_int >> c) & 1u) stack.push_back(nd.child_base + nd.meta[c]);
+            }
         }
         bool hit = best_gid != 0xFFFFFFFFu;
         if (hits) {
