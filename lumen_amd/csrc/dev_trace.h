@@ -26,6 +26,7 @@
 #include "bvh_layout.h"
 #include "context.h"
 #include "dev_math.h"
+#include "dev_work.h"
 
 namespace ltd {
 
@@ -370,90 +371,42 @@ LT_DEV bool trace_step(const SceneView& sv, TraceState& s, const TraceStack& stk
 }
 
 // Streams the queries [0, n_items) of a queue through one wave: every lane
-// steps its own query one node at a time, and lanes whose query finished
-// take new ones (one atomic per refill, refills once sv.refill_min lanes are
-// idle), so the wave stays full however uneven the traversal lengths are.
-// load(item, o, d, tmin, tmax) returns a tag handed to finish(tag, state).
-template <bool ANY, bool COUNT, class Load, class Finish>
+// steps its own query one node at a time, and once sv.refill_min lanes are
+// idle they hand out their results together and take new queries (one atomic
+// per refill), so the wave stays full however uneven the traversal lengths
+// are and nothing but the step runs between two refills.
+// load(item, o, d, tmin, tmax, any) returns a tag handed to finish(tag, state);
+// any says whether the query is an any-hit one (ANY_MASK 1: none is, 2: every
+// one is, 3: one by one).
+template <int ANY_MASK, bool COUNT, class Load, class Finish>
 LT_DEV void trace_stream(const SceneView& sv, const TraceStack& stk, uint32_t n_items, uint32_t* work, Load load,
                          Finish finish, uint32_t& n_nodes, uint32_t& n_tris) {
-    const uint32_t lane = threadIdx.x & 63u;
     TraceState s;
     uint32_t tag = 0;
-    bool has = false;
-    bool exhausted = false;  // wave-uniform
+    bool has = false, out = false, any = ANY_MASK == 2;
+    WaveTiles wt = wave_tiles(n_items, work);
     for (;;) {
-        if (!exhausted) {
-            const unsigned long long idle = __ballot(!has);
-            const uint32_t n_idle = (uint32_t)__popcll(idle);
-            if (n_idle >= sv.refill_min || n_idle == 64u) {
-                const int leader = __ffsll((long long)idle) - 1;
-                uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(work, n_idle);
-                base = __shfl(base, leader);
-                if (base + n_idle >= n_items) exhausted = true;
-                if (!has) {
-                    const uint32_t mine = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                    if (mine < n_items) {
-                        f3 o, d;
-                        float tmin, tmax;
-                        tag = load(mine, o, d, tmin, tmax);
-                        trace_init(sv, s, o, d, tmin, tmax);
-                        has = true;
-                    }
-                }
+        const unsigned long long idle = __ballot(!has);
+        const uint32_t n_idle = (uint32_t)__popcll(idle);
+        if (n_idle == 64u || (!wt.done && n_idle >= sv.refill_min)) {
+            if (out) finish(tag, s);
+            out = out && has;
+            if (n_idle == 64u && wt.done) break;
+            uint32_t item = 0u;
+            if (take_items(wt, idle, item)) {
+                f3 o, d;
+                float tmin, tmax;
+                bool a = ANY_MASK == 2;
+                tag = load(item, o, d, tmin, tmax, a);
+                if (ANY_MASK == 3) any = a;
+                trace_init(sv, s, o, d, tmin, tmax);
+                has = true;
             }
+            if (__ballot(has) == 0ull) break;
         }
-        if (__ballot(has) == 0ull) {
-            if (exhausted) break;
-            continue;
-        }
-        if (has && trace_step<ANY, COUNT>(sv, s, stk, n_nodes, n_tris)) {
-            finish(tag, s);
+        if (has && trace_step_dyn<COUNT>(sv, s, stk, ANY_MASK == 1 ? false : (ANY_MASK == 2 ? true : any), n_nodes, n_tris)) {
             has = false;
-        }
-    }
-}
-
-// trace_stream over a queue whose queries are closest-hit or any-hit one by
-// one: load(item, o, d, tmin, tmax, any) also says which.
-template <bool COUNT, class Load, class Finish>
-LT_DEV void trace_stream_mixed(const SceneView& sv, const TraceStack& stk, uint32_t n_items, uint32_t* work, Load load,
-                               Finish finish, uint32_t& n_nodes, uint32_t& n_tris) {
-    const uint32_t lane = threadIdx.x & 63u;
-    TraceState s;
-    uint32_t tag = 0;
-    bool has = false, any = false;
-    bool exhausted = false;  // wave-uniform
-    for (;;) {
-        if (!exhausted) {
-            const unsigned long long idle = __ballot(!has);
-            const uint32_t n_idle = (uint32_t)__popcll(idle);
-            if (n_idle >= sv.refill_min || n_idle == 64u) {
-                const int leader = __ffsll((long long)idle) - 1;
-                uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(work, n_idle);
-                base = __shfl(base, leader);
-                if (base + n_idle >= n_items) exhausted = true;
-                if (!has) {
-                    const uint32_t mine = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                    if (mine < n_items) {
-                        f3 o, d;
-                        float tmin, tmax;
-                        tag = load(mine, o, d, tmin, tmax, any);
-                        trace_init(sv, s, o, d, tmin, tmax);
-                        has = true;
-                    }
-                }
-            }
-        }
-        if (__ballot(has) == 0ull) {
-            if (exhausted) break;
-            continue;
-        }
-        if (has && trace_step_dyn<COUNT>(sv, s, stk, any, n_nodes, n_tris)) {
-            finish(tag, s);
-            has = false;
+            out = true;
         }
     }
 }

@@ -28,6 +28,7 @@ struct lt_integrator {
     lt_sppm_config sppm{};
     float4* accum = nullptr;  // output_tex, RGBA32F, row-major
     WaveBuffers wave;         // wavefront state (LT_PATH_WAVEFRONT)
+    PathSamples samples;      // sample radiance of multi-frame launches (LT_PATH_PERSISTENT)
     BdptBuffers bb;           // BDPT subpaths, camera estimates and splats
     VcmBuffers vb;            // VCM light vertices, photon grid and splats
     SppmBuffers sb;           // SPPM per-pixel state, photons and photon table
@@ -161,6 +162,7 @@ lt_status lt_integrator_destroy(lt_integrator* it) {
     if (it->ctx) (void)hipStreamSynchronize(it->ctx->stream);
     if (it->accum) (void)hipFree(it->accum);
     wave_free(it->wave);
+    path_samples_free(it->samples);
     bdpt_free(it->bb);
     vcm_free(it->vb);
     sppm_free(it->sb);
@@ -235,7 +237,7 @@ static lt_status launch_frames(lt_integrator* it, const lt_frame_params* p, uint
     if (it->path.strategy == LT_PATH_WAVEFRONT)
         return launch_path_wavefront(ctx, it->wave, L, it->accum, it->counting, ctx->count_buf);
     if (it->path.strategy == LT_PATH_PERSISTENT)
-        return launch_path_persistent(ctx, L, it->accum, it->counting, ctx->count_buf);
+        return launch_path_persistent(ctx, it->samples, L, it->accum, it->counting, ctx->count_buf);
     return launch_path_megakernel(ctx, L, it->accum, it->counting, ctx->count_buf);
 }
 

@@ -20,8 +20,23 @@ struct PathLaunch {
     const uint32_t* frame_dev;
     uint32_t regen_min;  // persistent kernel: idle lanes that trigger a refill
     uint32_t nee_pick;   // LT_NEE_REFERENCE or LT_NEE_CORRECTED
-    uint32_t xcd_bands;  // persistent kernel: pixels drawn per XCD from 8 bands
 };
+
+// Running mean of the accumulator (path.rgen:106-112).  The fused forms are
+// written out so that every kernel that accumulates rounds alike.
+LT_DEV void accumulate_mean(float4& acc, float r, float g, float b, uint32_t frame_num) {
+    if (frame_num > 0) {
+        const float w = 1.0f / (float)(frame_num + 1), k = 1.0f - w;
+        acc.x = fmaf(r, w, acc.x * k);
+        acc.y = fmaf(g, w, acc.y * k);
+        acc.z = fmaf(b, w, acc.z * k);
+    } else {
+        acc.x = r;
+        acc.y = g;
+        acc.z = b;
+    }
+    acc.w = 1.0f;
+}
 
 // Probability of the NEE light pick that sample_light_Li made (light `li`):
 // the reference's 1 / light_triangle_count (path.rgen:76-78), or
@@ -32,7 +47,16 @@ LT_DEV float nee_pick_pdf(const SceneView& sv, uint32_t nee_pick, uint32_t li) {
     return 1.0f / ((float)sv.num_lights * ((l.light_flags & 7u) == LT_LIGHT_AREA ? (float)l.num_triangles : 1.0f));
 }
 
-// persistent lanes with path regeneration, one launch per frame
-lt_status launch_path_persistent(lt_context* ctx, const PathLaunch& L, float4* accum, int count, uint64_t* d_counts);
+// Per-sample radiance of the frames of a multi-frame launch, [frame][pixel]
+// (w = 1, or 0 for a sample the NaN guard drops); kept by the integrator.
+struct PathSamples {
+    float4* rad = nullptr;
+    size_t capacity = 0;  // in float4
+};
+constexpr size_t kPathSampleBytes = 512ull << 20;  // frames of one launch: as many as fit
+void path_samples_free(PathSamples& s);
+// persistent lanes with path regeneration
+lt_status launch_path_persistent(lt_context* ctx, PathSamples& ps, const PathLaunch& L, float4* accum, int count,
+                                 uint64_t* d_counts);
 lt_status launch_path_megakernel(lt_context* ctx, const PathLaunch& L, float4* accum, int count,
                                  uint64_t* d_counts);

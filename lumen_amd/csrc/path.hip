@@ -7,6 +7,8 @@
 // src/shaders/integrators/pt_commons.glsl:3-47.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "context.h"
 #include "dev_scene.h"
 #include "dev_atmosphere.h"
@@ -138,11 +140,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     const uint32_t tiles_x = (L.width + 7) / 8, tiles_y = (L.height + 7) / 8;
     const uint32_t n_tiles = tiles_x * tiles_y;
     Ctr c{0, 0, 0, 0};
-    for (;;) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(work, 1u);
-        t = __shfl(t, 0);
-        if (t >= n_tiles) break;
+    WaveTiles wt = wave_tiles(n_tiles * 64u, work);
+    while (next_tile(wt)) {
+        const uint32_t t = wt.base >> 6;
         const uint32_t x = (t % tiles_x) * 8 + (lane & 7), y = (t / tiles_x) * 8 + (lane >> 3);
         if (x >= L.width || y >= L.height) continue;
         const size_t pix = (size_t)y * L.width + x;
@@ -152,17 +152,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
             const uint32_t frame_num = frame0 + f;
             f3 col;
             if (!path_sample<COUNT>(sv, L, x, y, frame_num ^ L.seed, stk, col, c)) continue;  // path.rgen:102-104
-            if (frame_num > 0) {
-                const float w = 1.0f / (float)(frame_num + 1);
-                acc.x = acc.x * (1.0f - w) + col.x * w;
-                acc.y = acc.y * (1.0f - w) + col.y * w;
-                acc.z = acc.z * (1.0f - w) + col.z * w;
-            } else {
-                acc.x = col.x;
-                acc.y = col.y;
-                acc.z = col.z;
-            }
-            acc.w = 1.0f;
+            accumulate_mean(acc, col.x, col.y, col.z, frame_num);
         }
         accum[pix] = acc;
     }
@@ -170,87 +160,81 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
 }
 
 // Path regeneration (the persistent form): each lane runs one bounce of its
-// path per iteration and, once the path ends, takes the next pixel of the
-// frame (a ballot over the idle lanes and one atomic per refill), so paths
+// path per iteration and, once the path ends, takes the next sample, so paths
 // of uneven length (Russian roulette, escapes) never leave lanes idle until
 // the longest path of a tile ends.  Per path the arithmetic, the RNG stream
 // and the result are those of path_sample.
+//
+// The items are the samples of L.spp frames, tile by tile of 8x8 pixels and a
+// tile's frames one after another: the frames share one launch, so the chip
+// drains once and not once per frame, and an image of fewer pixels than the
+// chip has lanes still fills it.  With one frame a sample goes straight into
+// the running mean; with more it goes to `rad` and k_path_mean folds a pixel's
+// samples in frame order.  16 frames of the 1080p terrain with a launch and a
+// contended counter each: 57.0 ms, in one launch 48.1 ms; of a 509 x 383 Cornell
+// box 4.2 (a wave per tile and its 16 samples in lockstep) and 1.8 ms.
 template <bool COUNT>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_PATH_MEGA_WAVES))) void k_path_regen(
-    SceneView sv, PathLaunch L, float4* __restrict__ accum, uint32_t* __restrict__ work, uint32_t* __restrict__ spill,
-    unsigned long long* __restrict__ counts) {
+    SceneView sv, PathLaunch L, float4* __restrict__ accum, float4* __restrict__ rad, uint32_t* __restrict__ work,
+    uint32_t* __restrict__ spill, unsigned long long* __restrict__ counts) {
     __shared__ uint32_t s_stack[ltb::kLdsWords * kTraceBlock];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     TraceStack stk{s_stack + threadIdx.x, spill + (size_t)gtid * (ltb::kStackTotal - ltb::kLdsStack)};
-    const uint32_t lane = threadIdx.x & 63u;
     const uint32_t tiles_x = (L.width + 7) / 8, tiles_y = (L.height + 7) / 8;
-    const uint32_t n_items = tiles_x * tiles_y * 64u;  // pixels in 8x8-tile order
-    const uint32_t frame_num = L.frame_dev ? *L.frame_dev : L.frame_start;
-    const uint32_t frame_word = frame_num ^ L.seed;
+    const uint32_t n_items = tiles_x * tiles_y * L.spp * 64u;
+    const uint32_t frame0 = L.frame_dev ? *L.frame_dev : L.frame_start;
     Ctr c{0, 0, 0, 0};
     PathState p;
-    // XCD bands: workgroups are dealt to the 8 XCDs round-robin (blockIdx mod
-    // 8); with bands on, the pixels are cut into 8 contiguous bands of tiles
-    // with a counter each, and a wave takes pixels from its XCD's band, so the
-    // primary rays of one L2 share a compact image region; a wave whose band
-    // is used up helps the next band.  Off: one counter over every pixel.
-    const uint32_t n_bands = (L.xcd_bands && (gridDim.x & 7u) == 0u) ? 8u : 1u;
-    const uint32_t band_len = (n_items + n_bands - 1u) / n_bands;
-    uint32_t band = n_bands == 8u ? (blockIdx.x & 7u) : 0u, bands_done = 0;  // wave-uniform
-    bool has = false, exhausted = false;  // exhausted is wave-uniform
+    bool has = false;
+    WaveTiles wt = wave_tiles(n_items, work);
     for (;;) {
-        if (!exhausted) {
-            const unsigned long long idle = __ballot(!has);
-            const uint32_t n_idle = (uint32_t)__popcll(idle);
-            if (n_idle >= L.regen_min || n_idle == 64u) {
-                const int leader = __ffsll((long long)idle) - 1;
-                uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(work + band, n_idle);
-                base = __shfl(base, leader);
-                const uint32_t band_lo = band * band_len, band_hi = min(n_items, band_lo + band_len);
-                const uint32_t first = band_lo + base;
-                if (first + n_idle >= band_hi) {  // this band is used up: the next one, until all are
-                    band = band + 1u == n_bands ? 0u : band + 1u;
-                    if (++bands_done == n_bands) exhausted = true;
+        const unsigned long long idle = __ballot(!has);
+        const uint32_t n_idle = (uint32_t)__popcll(idle);
+        if (n_idle == 64u || (!wt.done && n_idle >= L.regen_min)) {
+            if (n_idle == 64u && wt.done) break;
+            uint32_t t = 0u;
+            if (take_items(wt, idle, t)) {
+                const uint32_t w = t & 63u;
+                uint32_t tile = t >> 6, f = 0u;
+                if (L.spp > 1u) {
+                    f = tile % L.spp;
+                    tile /= L.spp;
                 }
-                if (!has) {
-                    const uint32_t t = first + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                    if (t < band_hi) {
-                        const uint32_t tile = t >> 6, w = t & 63u;
-                        const uint32_t x = (tile % tiles_x) * 8 + (w & 7u), y = (tile / tiles_x) * 8 + (w >> 3);
-                        if (x < L.width && y < L.height) {
-                            path_start(L, x, y, frame_word, p);
-                            p.pix = y * L.width + x;
-                            has = true;
-                        }
-                    }
+                const uint32_t x = (tile % tiles_x) * 8 + (w & 7u), y = (tile / tiles_x) * 8 + (w >> 3);
+                if (x < L.width && y < L.height) {
+                    path_start(L, x, y, (frame0 + f) ^ L.seed, p);
+                    p.pix = f * (L.width * L.height) + y * L.width + x;
+                    has = true;
                 }
             }
         }
-        if (__ballot(has) == 0ull) {
-            if (exhausted) break;
-            continue;
-        }
         if (has && !path_bounce<COUNT>(sv, L, p, stk, c)) {
             has = false;
-            if (!isnan(luminance(p.col))) {  // path.rgen:102-112
+            const bool ok = !isnan(luminance(p.col));  // path.rgen:102-104
+            if (L.spp > 1u) {
+                rad[p.pix] = make_float4(p.col.x, p.col.y, p.col.z, ok ? 1.0f : 0.0f);
+            } else if (ok) {
                 float4 acc = accum[p.pix];
-                if (frame_num > 0) {
-                    const float w = 1.0f / (float)(frame_num + 1);
-                    acc.x = acc.x * (1.0f - w) + p.col.x * w;
-                    acc.y = acc.y * (1.0f - w) + p.col.y * w;
-                    acc.z = acc.z * (1.0f - w) + p.col.z * w;
-                } else {
-                    acc.x = p.col.x;
-                    acc.y = p.col.y;
-                    acc.z = p.col.z;
-                }
-                acc.w = 1.0f;
+                accumulate_mean(acc, p.col.x, p.col.y, p.col.z, frame0);
                 accum[p.pix] = acc;
             }
         }
     }
     if (COUNT) flush_counts(c, counts);
+}
+
+// folds the samples of a multi-frame launch into the running mean (HBM bound:
+// 16 B per sample)
+__global__ __launch_bounds__(256) void k_path_mean(const float4* __restrict__ rad, float4* __restrict__ accum,
+                                                   uint32_t n, uint32_t frame0, uint32_t frames) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    float4 acc = accum[i];
+    for (uint32_t f = 0; f < frames; f++) {
+        const float4 r = rad[(size_t)f * n + i];
+        if (r.w != 0.0f) accumulate_mean(acc, r.x, r.y, r.z, frame0 + f);
+    }
+    accum[i] = acc;
 }
 
 __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
@@ -260,49 +244,79 @@ __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
 
 }  // namespace
 
+// workgroups of a persistent kernel: the tuning's count, but no more than the
+// chip holds at once (the tiles dealt out beforehand must all be under way)
+static size_t path_blocks(lt_context* ctx, const void* kernel) {
+    return (size_t)ctx->num_cus * std::min(ctx->tuning.path_blocks_per_cu, resident_blocks(kernel, 0u));
+}
+
 lt_status launch_path_megakernel(lt_context* ctx, const PathLaunch& L, float4* accum, int count,
                                  uint64_t* d_counts) {
-    const size_t blocks = (size_t)ctx->num_cus * ctx->tuning.path_blocks_per_cu;
+    const size_t blocks = path_blocks(ctx, count ? reinterpret_cast<const void*>(&k_path_mega<true>)
+                                                 : reinterpret_cast<const void*>(&k_path_mega<false>));
     lt_status st = ensure_spill(ctx, blocks * kTraceBlock);
     if (st != LT_OK) return st;
     SceneView sv = make_scene_view(ctx);
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 4u);
+    const uint64_t items = (uint64_t)((L.width + 7) / 8) * ((L.height + 7) / 8) * 64;
+    const uint32_t grid = work_blocks(items, (uint32_t)blocks, kTraceBlock / 64);
+    if (work_counted(items, grid, kTraceBlock / 64))
+        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 1u);
     if (count) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)d_counts, 2u * kCountSlots);
     auto* cnt = (unsigned long long*)d_counts;
     phase_mark(ctx);
     if (count)
-        hipLaunchKernelGGL((k_path_mega<true>), dim3(blocks), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
+        hipLaunchKernelGGL((k_path_mega<true>), dim3(grid), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
                            ctx->counters, ctx->spill, cnt);
     else
-        hipLaunchKernelGGL((k_path_mega<false>), dim3(blocks), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
+        hipLaunchKernelGGL((k_path_mega<false>), dim3(grid), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
                            ctx->counters, ctx->spill, cnt);
     LT_HIP(ctx, hipGetLastError());
     return LT_OK;
 }
 
-lt_status launch_path_persistent(lt_context* ctx, const PathLaunch& L0, float4* accum, int count,
+void path_samples_free(PathSamples& s) {
+    if (s.rad) (void)hipFree(s.rad);
+    s = PathSamples{};
+}
+
+lt_status launch_path_persistent(lt_context* ctx, PathSamples& ps, const PathLaunch& L0, float4* accum, int count,
                                  uint64_t* d_counts) {
-    const size_t blocks = (size_t)ctx->num_cus * ctx->tuning.path_blocks_per_cu;
+    const size_t blocks = path_blocks(ctx, count ? reinterpret_cast<const void*>(&k_path_regen<true>)
+                                                 : reinterpret_cast<const void*>(&k_path_regen<false>));
     lt_status st = ensure_spill(ctx, blocks * kTraceBlock);
     if (st != LT_OK) return st;
     if (L0.frame_dev && L0.spp != 1) return lt_fail(ctx, LT_ERR_INVALID_ARG, "a captured frame renders one frame");
+    const size_t n = (size_t)L0.width * L0.height;
+    // frames per launch: what the sample buffer holds, and items that fit 32 bits
+    const size_t items = (size_t)((L0.width + 7) / 8) * ((L0.height + 7) / 8) * 64;
+    const uint32_t group = (uint32_t)std::max<size_t>(
+        1, std::min<size_t>({L0.spp, kPathSampleBytes / (n * sizeof(float4)), (1ull << 31) / items}));
+    if (group > 1 && ps.capacity < group * n) {
+        path_samples_free(ps);
+        LT_HIP(ctx, hipMalloc(&ps.rad, group * n * sizeof(float4)));
+        ps.capacity = group * n;
+    }
     SceneView sv = make_scene_view(ctx);
     auto* cnt = (unsigned long long*)d_counts;
     if (count) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)d_counts, 2u * kCountSlots);
     phase_mark(ctx);
-    for (uint32_t f = 0; f < L0.spp; f++) {  // the running mean needs the frames in order
+    for (uint32_t f = 0; f < L0.spp; f += group) {
         PathLaunch L = L0;
         L.frame_start = L0.frame_start + f;
-        L.spp = 1;
+        L.spp = std::min(group, L0.spp - f);
         L.regen_min = ctx->tuning.regen_min ? ctx->tuning.regen_min : 4u;
-        L.xcd_bands = ctx->tuning.xcd_bands == LT_XCD_BANDS_ON ? 1u : 0u;
-        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 8u);
+        const uint32_t grid = work_blocks(items * L.spp, (uint32_t)blocks, kTraceBlock / 64);
+        if (work_counted(items * L.spp, grid, kTraceBlock / 64))
+            hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 1u);
         if (count)
-            hipLaunchKernelGGL((k_path_regen<true>), dim3(blocks), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
-                               ctx->counters, ctx->spill, cnt);
+            hipLaunchKernelGGL((k_path_regen<true>), dim3(grid), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
+                               ps.rad, ctx->counters, ctx->spill, cnt);
         else
-            hipLaunchKernelGGL((k_path_regen<false>), dim3(blocks), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
-                               ctx->counters, ctx->spill, cnt);
+            hipLaunchKernelGGL((k_path_regen<false>), dim3(grid), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
+                               ps.rad, ctx->counters, ctx->spill, cnt);
+        if (L.spp > 1u)
+            hipLaunchKernelGGL(k_path_mean, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, ps.rad, accum,
+                               (uint32_t)n, L.frame_start, L.spp);
     }
     LT_HIP(ctx, hipGetLastError());
     return LT_OK;

@@ -347,7 +347,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
             }
         }
     };
-    trace_stream_mixed<COUNT>(sv, stk, n_ext + n_sh + n_mis, &ctl->work[stage][0], load, finish, n_nodes, n_tris);
+    trace_stream<3, COUNT>(sv, stk, n_ext + n_sh + n_mis, &ctl->work[stage][0], load, finish, n_nodes, n_tris);
     if (COUNT) {
         unsigned long long a = n_nodes, b = n_tris, sh = n_shr, mi = n_misr;
         for (int o = 32; o > 0; o >>= 1) {
@@ -450,17 +450,7 @@ __global__ __launch_bounds__(256) void k_wf_accumulate(PathLaunch L, uint32_t f,
     c.z += mc.z;
     if (isnan(luminance(mk3(c.x, c.y, c.z)))) return;
     float4 acc = accum[p];
-    if (frame_num > 0) {
-        const float w = 1.0f / (float)(frame_num + 1);
-        acc.x = acc.x * (1.0f - w) + c.x * w;
-        acc.y = acc.y * (1.0f - w) + c.y * w;
-        acc.z = acc.z * (1.0f - w) + c.z * w;
-    } else {
-        acc.x = c.x;
-        acc.y = c.y;
-        acc.z = c.z;
-    }
-    acc.w = 1.0f;
+    accumulate_mean(acc, c.x, c.y, c.z, frame_num);
     accum[p] = acc;
 }
 

@@ -1,6 +1,7 @@
 // trace.hip — raw closest-hit / any-hit kernels behind lt_trace_closest,
 // lt_trace_any and lt_trace_count (persistent waves pulling 64 rays at a time).
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 
 #include <algorithm>
 #include <mutex>
@@ -24,30 +25,31 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(SceneView sv, const lt_ra
     TraceStack stk{s_stack + threadIdx.x, spill + (size_t)gtid * spill_stride};
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t n_nodes = 0, n_tris = 0;
-    for (;;) {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(work, 64u);
-        base = __shfl(base, 0);
-        if (base >= n) break;
-        const uint32_t i = base + lane;
-        if (i < n) {
-            const lt_ray r = rays[i];
-            HitRec h;
-            const bool hit = trace_bvh<ANY, COUNT>(sv, ld3(r.org), ld3(r.dir), r.tmin, r.tmax, h, stk, n_nodes,
-                                                   n_tris);
-            if (ANY) {
-                ((uint8_t*)out)[i] = hit ? 1 : 0;
-            } else {
-                lt_hit o;
-                o.t = hit ? h.t : 0.0f;
-                o.prim = h.prim;
-                o.inst = h.inst;
-                o.u = hit ? h.u : 0.0f;
-                o.v = hit ? h.v : 0.0f;
-                ((lt_hit*)out)[i] = o;
-            }
+    auto load = [&](uint32_t i, f3& o, f3& d, float& tmin, float& tmax, bool&) {
+        const float4* r = (const float4*)(rays + i);
+        const float4 a = r[0], b = r[1];
+        o = mk3(a.x, a.y, a.z);
+        tmin = a.w;
+        d = mk3(b.x, b.y, b.z);
+        tmax = b.w;
+        return i;
+    };
+    auto finish = [&](uint32_t i, const TraceState& s) {
+        const HitRec& h = s.best;
+        const bool hit = h.gid != 0xFFFFFFFFu;
+        if (ANY) {
+            ((uint8_t*)out)[i] = hit ? 1 : 0;
+        } else {
+            lt_hit o;
+            o.t = hit ? h.t : 0.0f;
+            o.prim = h.prim;
+            o.inst = h.inst;
+            o.u = hit ? h.u : 0.0f;
+            o.v = hit ? h.v : 0.0f;
+            ((lt_hit*)out)[i] = o;
         }
-    }
+    };
+    trace_stream<ANY ? 2 : 1, COUNT>(sv, stk, n, work, load, finish, n_nodes, n_tris);
     if (COUNT) {
         unsigned long long a = n_nodes, b = n_tris;
         for (int o = 32; o > 0; o >>= 1) {
@@ -61,6 +63,11 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(SceneView sv, const lt_ra
     }
 }
 
+__global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = v;
+}
+
 constexpr uint32_t kSpillStride = ltb::kStackTotal - ltb::kLdsStack;
 
 }  // namespace
@@ -69,31 +76,33 @@ lt_status launch_trace(lt_context* ctx, const lt_ray* d_rays, size_t n, void* d_
                        uint64_t* d_counts) {
     if (n == 0) return LT_OK;
     if (n > 0xFFFFFFFFull - 64) return lt_fail(ctx, LT_ERR_INVALID_ARG, "too many rays in one call");
-    const size_t blocks = (size_t)ctx->num_cus * ctx->tuning.trace_blocks_per_cu;
-    lt_status st = ensure_spill(ctx, blocks * kTraceBlock);
+    const void* kernel = any_hit ? (count ? reinterpret_cast<const void*>(&k_trace<true, true>)
+                                          : reinterpret_cast<const void*>(&k_trace<true, false>))
+                                 : (count ? reinterpret_cast<const void*>(&k_trace<false, true>)
+                                          : reinterpret_cast<const void*>(&k_trace<false, false>));
+    // as many workgroups as the chip holds at once, or fewer where the rays are
+    const uint32_t most = (uint32_t)ctx->num_cus * std::min(ctx->tuning.trace_blocks_per_cu, resident_blocks(kernel, 0u));
+    lt_status st = ensure_spill(ctx, (size_t)most * kTraceBlock);
     if (st != LT_OK) return st;
+    const uint32_t blocks = work_blocks(n, most, kTraceBlock / 64);
     SceneView sv = make_scene_view(ctx);
-    LT_HIP(ctx, hipMemsetAsync(ctx->counters, 0, 4, ctx->stream));
-    if (count) LT_HIP(ctx, hipMemsetAsync(d_counts, 0, 16, ctx->stream));
-    LT_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+    if (work_counted(n, blocks, kTraceBlock / 64))
+        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 1u, 0u);
+    if (count) hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)d_counts, 4u, 0u);
     auto* cnt = (unsigned long long*)d_counts;
-    if (any_hit) {
-        if (count)
-            hipLaunchKernelGGL((k_trace<true, true>), dim3(blocks), dim3(kTraceBlock), 0, ctx->stream, sv, d_rays,
-                               (uint32_t)n, d_out, ctx->counters, ctx->spill, kSpillStride, cnt);
-        else
-            hipLaunchKernelGGL((k_trace<true, false>), dim3(blocks), dim3(kTraceBlock), 0, ctx->stream, sv, d_rays,
-                               (uint32_t)n, d_out, ctx->counters, ctx->spill, kSpillStride, cnt);
+    uint32_t n32 = (uint32_t)n, stride = kSpillStride;
+    void* args[] = {&sv, &d_rays, &n32, &d_out, &ctx->counters, &ctx->spill, &stride, &cnt};
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    LT_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cap));
+    if (cap == hipStreamCaptureStatusNone) {
+        // the events take the dispatch packet's own timestamps (a record
+        // before and after the kernel costs two more packets, several us each)
+        LT_HIP(ctx, hipExtLaunchKernel(kernel, dim3(blocks), dim3(kTraceBlock), args, 0, ctx->stream, ctx->ev0, ctx->ev1, 0));
     } else {
-        if (count)
-            hipLaunchKernelGGL((k_trace<false, true>), dim3(blocks), dim3(kTraceBlock), 0, ctx->stream, sv, d_rays,
-                               (uint32_t)n, d_out, ctx->counters, ctx->spill, kSpillStride, cnt);
-        else
-            hipLaunchKernelGGL((k_trace<false, false>), dim3(blocks), dim3(kTraceBlock), 0, ctx->stream, sv, d_rays,
-                               (uint32_t)n, d_out, ctx->counters, ctx->spill, kSpillStride, cnt);
+        LT_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+        LT_HIP(ctx, hipLaunchKernel(kernel, dim3(blocks), dim3(kTraceBlock), args, 0, ctx->stream));
+        LT_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     }
-    LT_HIP(ctx, hipGetLastError());
-    LT_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     return LT_OK;
 }
 
@@ -116,11 +125,6 @@ constexpr size_t kNoAllocWords = kNoAllocCounterWords + (size_t)kNoAllocBlocks *
 
 // 8 MiB + 256 B per device, held until the process ends
 __device__ __align__(256) uint32_t scratch[kNoAllocWords];
-
-__global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -156,7 +160,10 @@ extern "C" lt_status lt_trace_closest_noalloc(lt_context* ctx, const lt_ray* ray
                            " exceeds the " + std::to_string(ltb::kLdsStack + kNoAllocSpill + 1) +
                            " levels its fixed stack holds");
     LT_HIP(ctx, hipSetDevice(ctx->device));
-    const size_t blocks = std::min<size_t>((size_t)ctx->num_cus * ctx->tuning.trace_blocks_per_cu, kNoAllocBlocks);
+    const void* kernel = reinterpret_cast<const void*>(&k_trace<false, false>);
+    const uint32_t blocks = work_blocks(
+        n, std::min((uint32_t)ctx->num_cus * std::min(ctx->tuning.trace_blocks_per_cu, resident_blocks(kernel, 0u)),
+                    kNoAllocBlocks), kTraceBlock / 64);
     uint32_t* work = ctx->noalloc_scratch;
     uint32_t* spill = work + kNoAllocCounterWords;
     SceneView sv = make_scene_view(ctx);
