@@ -594,8 +594,8 @@ def main() -> int:
     else:
         workload = "terrain-1M+2000-boxes-1920x1080-path-d12"
         out_integrator = f"path-{args.strategy}"
-        roof = line("k_path_mega" if args.strategy == "megakernel" else
-                    "k_path_regen (one launch per frame)" if args.strategy == "persistent" else
+        roof = line(
+                    "k_path_regen (one launch per frame)" if args.strategy != "wavefront" else
                     "one frame's launch sequence (trace + shade per depth)", bvh_bytes, avg_ms)
     roof["traffic"] = traffic_from_profile(workload, out_integrator)
 

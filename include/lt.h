@@ -293,11 +293,12 @@ lt_status lt_trace_count(lt_context* ctx, const lt_ray* rays, size_t n, int any_
  * keeps the current value).  Set by the autotuner (lumen_amd/autotune.py).
  * No reference counterpart: the reference's launch shapes are the driver's. */
 typedef struct lt_tuning {
-    uint32_t path_blocks_per_cu;   /* Path megakernel and wavefront trace stages, 128-thread
-                                      workgroups (default 10)                           */
-    uint32_t trace_blocks_per_cu;  /* raw queries, 128-thread workgroups (default 8)     */
-    uint32_t refill_min;           /* wavefront trace stages: idle lanes that trigger a
-                                      refill from the queue, 1..64 (default 32)         */
+    uint32_t path_blocks_per_cu;   /* Path kernel and wavefront trace stages, 128-thread
+                                      workgroups (default 10), at most what a CU holds  */
+    uint32_t trace_blocks_per_cu;  /* raw queries, 128-thread workgroups (default 8), at
+                                      most what a CU holds                              */
+    uint32_t refill_min;           /* raw queries and wavefront trace stages: idle lanes
+                                      that trigger a refill, 1..64 (default 32)         */
     uint32_t bdpt_blocks_per_cu;   /* BDPT and VCM persistent kernels, 128-thread
                                       workgroups; default 0 = each kernel's resident
                                       workgroups per CU (its register and LDS use).
@@ -311,10 +312,9 @@ typedef struct lt_tuning {
                                       (default) or LT_WF_SORT_BSDF (the hit paths of a
                                       depth grouped by the BSDF type of their material
                                       before shading); 0 = unchanged                     */
-    uint32_t xcd_bands;            /* persistent Path kernel: LT_XCD_BANDS_OFF (default) or
-                                      LT_XCD_BANDS_ON (the pixels cut into 8 bands, one
-                                      per XCD's workgroups, each with its own counter);
-                                      0 = unchanged                                      */
+    uint32_t xcd_bands;            /* LT_XCD_BANDS_OFF (default) or LT_XCD_BANDS_ON; kept
+                                      and returned, no effect: the tiles of a round are
+                                      always dealt in one run per XCD; 0 = unchanged     */
     uint32_t reserved[8];
 } lt_tuning;
 #define LT_WF_SORT_NONE 1u
@@ -350,7 +350,8 @@ typedef enum lt_integrator_kind {
 } lt_integrator_kind;
 
 /* Path execution strategies. */
-#define LT_PATH_MEGAKERNEL 0u /* one thread per pixel, whole path in one kernel */
+#define LT_PATH_MEGAKERNEL 0u /* whole path in one kernel; runs as LT_PATH_PERSISTENT,
+                                 which is as fast for one frame and faster for several */
 #define LT_PATH_WAVEFRONT 1u  /* persistent stages with compacted ray queues   */
 #define LT_PATH_PERSISTENT 2u /* persistent lanes with path regeneration: a lane
                                  takes the next pixel as soon as its path ends */

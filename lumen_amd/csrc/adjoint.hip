@@ -2,7 +2,7 @@
 // adjoint on gfx950.
 //
 // No reference counterpart (the reference renders but does not
-// differentiate).  The estimator is the Path megakernel's per-sample logic
+// differentiate).  The estimator is the Path kernel's per-sample logic
 // (src/shaders/integrators/path/path.rgen:26-104, pt_commons.glsl:3-42)
 // without roulette; the albedo and roughness textures aid / rid are read
 // from per-variant texel arrays.  Derivatives hold the random numbers fixed

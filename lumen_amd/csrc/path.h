@@ -58,5 +58,3 @@ void path_samples_free(PathSamples& s);
 // persistent lanes with path regeneration
 lt_status launch_path_persistent(lt_context* ctx, PathSamples& ps, const PathLaunch& L, float4* accum, int count,
                                  uint64_t* d_counts);
-lt_status launch_path_megakernel(lt_context* ctx, const PathLaunch& L, float4* accum, int count,
-                                 uint64_t* d_counts);

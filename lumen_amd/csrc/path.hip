@@ -1,4 +1,4 @@
-// path.hip — the Path integrator on gfx950 (megakernel form).
+// path.hip — the Path integrator on gfx950 (persistent form).
 //
 // One thread per pixel, persistent waves pulling 8x8 pixel tiles, all frames
 // of a launch accumulated in registers with the reference's per-frame running
@@ -108,56 +108,12 @@ LT_DEV bool path_bounce(const SceneView& sv, const PathLaunch& L, PathState& p, 
     return alive;
 }
 
-// One path of pixel (x, y) (path.rgen:26-104); false when the NaN guard
-// drops the sample.
-template <bool COUNT>
-LT_DEV bool path_sample(const SceneView& sv, const PathLaunch& L, uint32_t x, uint32_t y, uint32_t frame_word,
-                        const TraceStack& stk, f3& col, Ctr& c) {
-    PathState p;
-    path_start(L, x, y, frame_word, p);
-    while (path_bounce<COUNT>(sv, L, p, stk, c)) {
-    }
-    col = p.col;
-    return !isnan(luminance(col));
-}
-
-template <bool COUNT>
 // Four waves per SIMD (128 VGPRs; the path state across a traversal spills to
 // scratch, which stays in cache): 6.5 ms per 1080p terrain frame against
-// 9.0 ms at the unconstrained 203 VGPRs / 2 waves.  A cap of five waves
-// (96 VGPRs, 416 B of scratch per lane) produced wrong images with no cause
-// found in this source, so it is not used.
+// 9.0 ms at the unconstrained 203 VGPRs / 2 waves, in an earlier form.
 #ifndef LT_PATH_MEGA_WAVES
 #define LT_PATH_MEGA_WAVES 4
 #endif
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_PATH_MEGA_WAVES))) void k_path_mega(SceneView sv, PathLaunch L, float4* __restrict__ accum,
-                                                           uint32_t* __restrict__ work, uint32_t* __restrict__ spill,
-                                                           unsigned long long* __restrict__ counts) {
-    __shared__ uint32_t s_stack[ltb::kLdsWords * kTraceBlock];
-    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    TraceStack stk{s_stack + threadIdx.x, spill + (size_t)gtid * (ltb::kStackTotal - ltb::kLdsStack)};
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t tiles_x = (L.width + 7) / 8, tiles_y = (L.height + 7) / 8;
-    const uint32_t n_tiles = tiles_x * tiles_y;
-    Ctr c{0, 0, 0, 0};
-    WaveTiles wt = wave_tiles(n_tiles * 64u, work);
-    while (next_tile(wt)) {
-        const uint32_t t = wt.base >> 6;
-        const uint32_t x = (t % tiles_x) * 8 + (lane & 7), y = (t / tiles_x) * 8 + (lane >> 3);
-        if (x >= L.width || y >= L.height) continue;
-        const size_t pix = (size_t)y * L.width + x;
-        float4 acc = accum[pix];
-        const uint32_t frame0 = L.frame_dev ? *L.frame_dev : L.frame_start;
-        for (uint32_t f = 0; f < L.spp; f++) {
-            const uint32_t frame_num = frame0 + f;
-            f3 col;
-            if (!path_sample<COUNT>(sv, L, x, y, frame_num ^ L.seed, stk, col, c)) continue;  // path.rgen:102-104
-            accumulate_mean(acc, col.x, col.y, col.z, frame_num);
-        }
-        accum[pix] = acc;
-    }
-    if (COUNT) flush_counts(c, counts);
-}
 
 // Path regeneration (the persistent form): each lane runs one bounce of its
 // path per iteration and, once the path ends, takes the next sample, so paths
@@ -248,30 +204,6 @@ __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
 // chip holds at once (the tiles dealt out beforehand must all be under way)
 static size_t path_blocks(lt_context* ctx, const void* kernel) {
     return (size_t)ctx->num_cus * std::min(ctx->tuning.path_blocks_per_cu, resident_blocks(kernel, 0u));
-}
-
-lt_status launch_path_megakernel(lt_context* ctx, const PathLaunch& L, float4* accum, int count,
-                                 uint64_t* d_counts) {
-    const size_t blocks = path_blocks(ctx, count ? reinterpret_cast<const void*>(&k_path_mega<true>)
-                                                 : reinterpret_cast<const void*>(&k_path_mega<false>));
-    lt_status st = ensure_spill(ctx, blocks * kTraceBlock);
-    if (st != LT_OK) return st;
-    SceneView sv = make_scene_view(ctx);
-    const uint64_t items = (uint64_t)((L.width + 7) / 8) * ((L.height + 7) / 8) * 64;
-    const uint32_t grid = work_blocks(items, (uint32_t)blocks, kTraceBlock / 64);
-    if (work_counted(items, grid, kTraceBlock / 64))
-        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 1u);
-    if (count) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)d_counts, 2u * kCountSlots);
-    auto* cnt = (unsigned long long*)d_counts;
-    phase_mark(ctx);
-    if (count)
-        hipLaunchKernelGGL((k_path_mega<true>), dim3(grid), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
-                           ctx->counters, ctx->spill, cnt);
-    else
-        hipLaunchKernelGGL((k_path_mega<false>), dim3(grid), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
-                           ctx->counters, ctx->spill, cnt);
-    LT_HIP(ctx, hipGetLastError());
-    return LT_OK;
 }
 
 void path_samples_free(PathSamples& s) {

@@ -15,7 +15,7 @@
 // Terminated paths leave the queues (ballot + one atomic per wave), so every
 // stage runs on full waves whatever the path lengths.  Each path consumes its
 // pcg4d stream in exactly the order of path.rgen / pt_commons.glsl, so the
-// image equals the megakernel's up to float summation order.
+// image equals the persistent kernel's up to float summation order.
 #include <hip/hip_runtime.h>
 
 #include "context.h"
