@@ -23,7 +23,18 @@ struct VcmLaunch {
     float sky_col[3];
     uint32_t use_vm;
     uint32_t corrected;  // 0: the reference estimator, 1: corrected VCM
+    uint32_t regen_min;  // light pass: idle lanes that trigger taking new paths
 };
+
+// The merge queries lie in segments, one counter each, on cache lines of their
+// own; tile t of the image writes segment t mod kQuerySegs.
+constexpr uint32_t kQuerySegs = 64;
+constexpr uint32_t kQueryCtrStride = 32;  // words between counters
+constexpr uint32_t kMergeTasks = 16384;   // merge tasks a segment's list holds
+__host__ __device__ inline size_t query_seg_cap(const VcmLaunch& L) {
+    const size_t tiles = (size_t)((L.width + 7) / 8) * ((L.height + 7) / 8);
+    return (tiles + kQuerySegs - 1) / kQuerySegs * 64 * (size_t)L.max_depth;
+}
 
 // A merge query of the corrected estimator, 80 B: an eye vertex and the
 // camera subpath state merging needs, written by the eye pass and gathered
@@ -43,7 +54,7 @@ struct VcmVertex {
     float4 c;  // wi.xyz, d_vm
     float4 d;  // wo.xyz, uv.x
     float4 e;  // throughput.xyz, uv.y
-    uint4 f;   // material_idx, path_len, side, 0
+    uint4 f;   // material_idx, path_len, side, rank in its photon bucket (corrected estimator)
 };
 
 // A photon of the corrected estimator's bucketed list: its position (and
@@ -72,7 +83,6 @@ struct VcmBuffers {
     uint32_t* key = nullptr;
     uint32_t* count = nullptr;
     uint32_t* start = nullptr;
-    uint32_t* fill = nullptr;
     float4* ppos = nullptr;  // pos.xyz, d_vcm
     VcmPhotonRest* prest = nullptr;
     void* scan_tmp = nullptr;
@@ -82,7 +92,8 @@ struct VcmBuffers {
     // by the merge pass) and its merge queries (at most max_depth per pixel)
     float4* fcol = nullptr;
     VcmQuery* queries = nullptr;
-    uint32_t* qctr = nullptr;  // queries written
+    uint2* tasks = nullptr;    // parts of heavy merge queries: query of the segment, part
+    uint32_t* qctr = nullptr;  // queries written, then tasks listed, per segment
     uint32_t n_paths = 0;
     int32_t max_depth = 0;
 };

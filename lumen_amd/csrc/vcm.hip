@@ -10,7 +10,8 @@
 //                 reference inserted (atomicMax, a deterministic "last
 //                 writer") and the insertion count; corrected estimator: an
 //                 exclusive scan of the bucket counts and a scatter of every
-//                 photon (k_vcm_scatter: 16-B positions, 48-B rest);
+//                 photon (k_vcm_scatter: 16-B positions, 48-B rest) to its
+//                 rank in the bucket, which the light pass's count returned;
 //   k_vcm_eye     one camera path per pixel (vcm_eye.rgen:42-98,
 //                 vcm_commons.glsl:477-631): emission, NEE, connections to the
 //                 vertices of one random light path; the reference estimator
@@ -97,6 +98,20 @@ LT_DEV void grid_idx_fast(const VcmLaunch& L, f3 p, int o[3]) {
     o[2] = (int)((p.z - L.bmin[2]) * L.inv_ext[2] * (float)L.grid_res[2]);
 }
 
+// The corrected estimator's buckets: 8 cells that follow one another along z
+// share a run of 8 buckets, and the runs are hashed.  A query's box of 5^3 cells
+// then is 25 columns of one or two contiguous bucket ranges each, so one
+// step of a wave reads all its ranges (64 lanes, two words each) where a bucket
+// per cell took two steps of 64 scattered ones.
+constexpr int kRunBits = 3;
+LT_DEV uint32_t run_base(int x, int y, int run, uint32_t n) {
+    const uint32_t h = ((uint32_t)x * 73856093u) ^ ((uint32_t)y * 19349663u) ^ ((uint32_t)run * 83492791u);
+    return (h % ((10u * n) >> kRunBits)) << kRunBits;
+}
+LT_DEV uint32_t run_bucket(const int g[3], uint32_t n) {
+    return run_base(g[0], g[1], g[2] >> kRunBits, n) + ((uint32_t)g[2] & ((1u << kRunBits) - 1u));
+}
+
 template <bool COUNT>
 LT_DEV bool occluded(const SceneView& sv, f3 o, f3 d, float tmax, const TraceStack& stk, Ctr& c) {
     if (COUNT) c.shadow++;
@@ -165,11 +180,17 @@ LT_DEV int connect_cam(const SceneView& sv, const VcmLaunch& L, const Camera& ca
     return (int)fy * (int)L.width + (int)fx;
 }
 
-template <bool COUNT>
-LT_DEV uint32_t light_path(const SceneView& sv, const VcmLaunch& L, const Camera& cam, uint32_t p,
-                           VcmVertex* __restrict__ lv, float* __restrict__ splat, const TraceStack& stk, Ctr& c) {
-    const uint32_t x = p / L.height, y = p % L.height;  // pixel_idx = x * H + y (vcm_light.rgen:56)
-    RNG seed = {x, y, L.light_word, 0u};
+// A light subpath between two bounces (vcm_light.rgen:123-166).
+struct LightState {
+    VState st;
+    uint32_t p, rng;   // path (pixel slot), RNG counter
+    uint32_t depth, n; // next bounce, stored vertices
+    bool finite;       // of a finite light
+};
+
+// false if the light has no emission sample
+LT_DEV bool light_begin(const SceneView& sv, const VcmLaunch& L, uint32_t p, LightState& s) {
+    RNG seed = {p / L.height, p % L.height, L.light_word, 0u};  // pixel_idx = x * H + y (vcm_light.rgen:56)
     f4 rp;
     rp.x = rnd(seed);
     rp.y = rnd(seed);
@@ -180,83 +201,110 @@ LT_DEV uint32_t light_path(const SceneView& sv, const VcmLaunch& L, const Camera
     uint32_t flags, li;
     f3 pos, wi, n;
     const f3 Le = sample_light_Le(sv, rp, rd0, rd1, cos_theta, flags, li, pos, wi, n, pdf_pos, pdf_dir);
-    if (pdf_dir <= 0.0f) return 0;
-    VState st;
+    s.p = p;
+    s.rng = seed.w;
+    s.depth = 1u;
+    s.n = 0u;
+    if (pdf_dir <= 0.0f) return false;
+    VState& st = s.st;
     const float pdf_emit = pdf_pos * pdf_dir, pdf_direct = pdf_pos;
     st.pos = pos;
     st.wi = wi;
     st.n_s = n;
     st.thr = Le * cos_theta / (pdf_dir * pdf_pos);
     st.d_vcm = pdf_direct / pdf_emit;
-    const bool finite = light_finite(flags);
-    st.d_vc = light_delta(flags) ? 0.0f : (finite ? cos_theta : 1.0f) / (pdf_dir * pdf_pos);
+    s.finite = light_finite(flags);
+    st.d_vc = light_delta(flags) ? 0.0f : (s.finite ? cos_theta : 1.0f) / (pdf_dir * pdf_pos);
     st.d_vm = st.d_vc * L.eta_vc;
-    uint32_t path_idx = 0;
-    for (int depth = 1;; depth++) {
-        Payload pl;
-        if (!closest<COUNT>(sv, st.pos, st.wi, pl, stk, c)) break;
-        f3 wo = st.pos - pl.pos;
-        f3 n_s = pl.n_s, n_g = pl.n_g;
-        bool side = true;
-        if (dot(pl.n_g, wo) <= 0.0f) n_g = -n_g;
-        if (dot(n_g, n_s) < 0.0f) {
-            n_s = -n_s;
-            side = false;
-        }
-        const float dist = length(pl.pos - st.pos);
-        const float dist_sqr = dist * dist;
-        wo /= dist;
-        const Mat mat = load_material(sv, pl.material_idx, pl.uv);
-        const bool spec = (mat.bsdf_props & LT_BSDF_FLAG_SPECULAR) == LT_BSDF_FLAG_SPECULAR;
-        const float cos_theta_wo = fabsf(dot(wo, n_s));
-        if (depth > 1 || finite) st.d_vcm *= dist_sqr;
-        st.d_vcm /= cos_theta_wo;
-        st.d_vc /= cos_theta_wo;
-        st.d_vm /= cos_theta_wo;
-        if (!spec) {  // vertex connection is always on (VCM.cpp:7)
-            VcmVertex* v = lv + path_idx;
-            v->a = make_float4(pl.pos.x, pl.pos.y, pl.pos.z, st.d_vcm);
-            v->b = make_float4(n_s.x, n_s.y, n_s.z, st.d_vc);
-            v->c = make_float4(st.wi.x, st.wi.y, st.wi.z, st.d_vm);
-            v->d = make_float4(wo.x, wo.y, wo.z, pl.uv.x);
-            v->e = make_float4(st.thr.x, st.thr.y, st.thr.z, pl.uv.y);
-            v->f = make_uint4(pl.material_idx, (uint32_t)depth + 1u, side ? 1u : 0u, 0u);
-            path_idx++;
-        }
-        if (depth >= L.max_depth) break;
-        if (!spec) {
-            f3 sc;
-            const int px = connect_cam<COUNT>(sv, L, cam, n_s, pl.n_s, pl.pos, st, wo, mat, sc, stk, c);
-            if (px >= 0) {
-                float* dst = splat + 3 * (size_t)px;
-                unsafeAtomicAdd(dst, sc.x);
-                unsafeAtomicAdd(dst + 1, sc.y);
-                unsafeAtomicAdd(dst + 2, sc.z);
+    return true;
+}
+
+// One bounce (vcm_commons.glsl:302-474); false once the path has ended.
+template <bool COUNT>
+LT_DEV bool light_step(const SceneView& sv, const VcmLaunch& L, const Camera& cam, LightState& s,
+                       VcmVertex* __restrict__ verts, float* __restrict__ splat, uint32_t* __restrict__ key,
+                       uint32_t* __restrict__ count, const TraceStack& stk, Ctr& c) {
+    VState& st = s.st;
+    const int depth = (int)s.depth++;
+    Payload pl;
+    if (!closest<COUNT>(sv, st.pos, st.wi, pl, stk, c)) return false;
+    f3 wo = st.pos - pl.pos;
+    f3 n_s = pl.n_s, n_g = pl.n_g;
+    bool side = true;
+    if (dot(pl.n_g, wo) <= 0.0f) n_g = -n_g;
+    if (dot(n_g, n_s) < 0.0f) {
+        n_s = -n_s;
+        side = false;
+    }
+    const float dist = length(pl.pos - st.pos);
+    const float dist_sqr = dist * dist;
+    wo /= dist;
+    const Mat mat = load_material(sv, pl.material_idx, pl.uv);
+    const bool spec = (mat.bsdf_props & LT_BSDF_FLAG_SPECULAR) == LT_BSDF_FLAG_SPECULAR;
+    const float cos_theta_wo = fabsf(dot(wo, n_s));
+    if (depth > 1 || s.finite) st.d_vcm *= dist_sqr;
+    st.d_vcm /= cos_theta_wo;
+    st.d_vc /= cos_theta_wo;
+    st.d_vm /= cos_theta_wo;
+    if (!spec) {  // vertex connection is always on (VCM.cpp:7)
+        const uint32_t ref = s.p * ((uint32_t)L.max_depth + 1u) + s.n;
+        uint32_t rank = 0u;
+        if (L.use_vm) {  // vcm_commons.glsl:455-469
+            int g[3];
+            if (L.corrected) {
+                grid_idx_fast(L, pl.pos, g);
+                rank = atomicAdd(&count[run_bucket(g, L.n_paths)], 1u);
+            } else {
+                grid_idx(L, pl.pos, g);
+                const uint32_t h = cell_hash(g[0], g[1], g[2], L.n_paths);
+                atomicMax(&key[h], ref + 1u);
+                atomicAdd(&count[h], 1u);
             }
         }
-        float pdf_d, cos_t;
-        const float r0 = rnd(seed), r1 = rnd(seed), r2 = rnd(seed);
-        const f3 f = sample_bsdf(n_s, wo, mat, 0u, side, st.wi, pdf_d, cos_t, r0, r1, r2);
-        const bool same_hem = dot(st.wi, n_s) > 0.0f && dot(wo, n_s) > 0.0f;
-        const bool transm = (mat.bsdf_props & LT_BSDF_FLAG_TRANSMISSION) == LT_BSDF_FLAG_TRANSMISSION;
-        if (is_zero(f) || pdf_d == 0.0f || (!same_hem && !transm)) break;
-        float pdf_rev = pdf_d;
-        if (!spec) pdf_rev = bsdf_pdf(mat, n_s, st.wi, wo, side);
-        const float ac = fabsf(cos_t);
-        st.pos = offset_ray(pl.pos, n_g);
-        if (!spec) {
-            st.d_vc = (ac / pdf_d) * (L.eta_vm + st.d_vcm + pdf_rev * st.d_vc);
-            st.d_vm = (ac / pdf_d) * (1.0f + st.d_vcm * L.eta_vc + pdf_rev * st.d_vm);
-            st.d_vcm = 1.0f / pdf_d;
-        } else {
-            st.d_vcm = 0.0f;
-            st.d_vc *= ac;
-            st.d_vm *= ac;
-        }
-        st.thr *= f * ac / pdf_d;
-        st.n_s = n_s;
+        VcmVertex* v = verts + ref;
+        v->a = make_float4(pl.pos.x, pl.pos.y, pl.pos.z, st.d_vcm);
+        v->b = make_float4(n_s.x, n_s.y, n_s.z, st.d_vc);
+        v->c = make_float4(st.wi.x, st.wi.y, st.wi.z, st.d_vm);
+        v->d = make_float4(wo.x, wo.y, wo.z, pl.uv.x);
+        v->e = make_float4(st.thr.x, st.thr.y, st.thr.z, pl.uv.y);
+        v->f = make_uint4(pl.material_idx, (uint32_t)depth + 1u, side ? 1u : 0u, rank);
+        s.n++;
     }
-    return path_idx;
+    if (depth >= L.max_depth) return false;
+    if (!spec) {
+        f3 sc;
+        const int px = connect_cam<COUNT>(sv, L, cam, n_s, pl.n_s, pl.pos, st, wo, mat, sc, stk, c);
+        if (px >= 0) {
+            float* dst = splat + 3 * (size_t)px;
+            unsafeAtomicAdd(dst, sc.x);
+            unsafeAtomicAdd(dst + 1, sc.y);
+            unsafeAtomicAdd(dst + 2, sc.z);
+        }
+    }
+    float pdf_d, cos_t;
+    RNG seed = {s.p / L.height, s.p % L.height, L.light_word, s.rng};
+    const float r0 = rnd(seed), r1 = rnd(seed), r2 = rnd(seed);
+    s.rng = seed.w;
+    const f3 f = sample_bsdf(n_s, wo, mat, 0u, side, st.wi, pdf_d, cos_t, r0, r1, r2);
+    const bool same_hem = dot(st.wi, n_s) > 0.0f && dot(wo, n_s) > 0.0f;
+    const bool transm = (mat.bsdf_props & LT_BSDF_FLAG_TRANSMISSION) == LT_BSDF_FLAG_TRANSMISSION;
+    if (is_zero(f) || pdf_d == 0.0f || (!same_hem && !transm)) return false;
+    float pdf_rev = pdf_d;
+    if (!spec) pdf_rev = bsdf_pdf(mat, n_s, st.wi, wo, side);
+    const float ac = fabsf(cos_t);
+    st.pos = offset_ray(pl.pos, n_g);
+    if (!spec) {
+        st.d_vc = (ac / pdf_d) * (L.eta_vm + st.d_vcm + pdf_rev * st.d_vc);
+        st.d_vm = (ac / pdf_d) * (1.0f + st.d_vcm * L.eta_vc + pdf_rev * st.d_vm);
+        st.d_vcm = 1.0f / pdf_d;
+    } else {
+        st.d_vcm = 0.0f;
+        st.d_vc *= ac;
+        st.d_vm *= ac;
+    }
+    st.thr *= f * ac / pdf_d;
+    st.n_s = n_s;
+    return true;
 }
 
 // Three waves per SIMD (168 VGPRs, no scratch); four (128 VGPRs, 148 B of
@@ -275,33 +323,27 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     __shared__ uint32_t s_stack[ltb::kLdsWords * kTraceBlock];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     TraceStack stk{s_stack + threadIdx.x, spill + (size_t)gtid * (ltb::kStackTotal - ltb::kLdsStack)};
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t chunks = (L.n_paths + 63u) / 64u;
-    const uint32_t nv = (uint32_t)L.max_depth + 1u;
     const Camera cam = camera_of(L);
     Ctr c{0, 0, 0, 0};
+    // a lane takes the next path as soon as its own ends (one bounce per
+    // iteration), so a wave does not wait for the longest path of 64
+    LightState s;
+    bool has = false;
+    WaveTiles wt = wave_tiles(L.n_paths, work);
     for (;;) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(work, 1u);
-        t = __shfl(t, 0);
-        if (t >= chunks) break;
-        const uint32_t p = t * 64u + lane;
-        if (p >= L.n_paths) continue;
-        VcmVertex* lv = verts + (size_t)p * nv;
-        const uint32_t n = light_path<COUNT>(sv, L, cam, p, lv, splat, stk, c);
-        cnt[p] = n;
-        if (L.use_vm) {  // vcm_commons.glsl:455-469
-            for (uint32_t i = 0; i < n; i++) {
-                const float4 a = lv[i].a;
-                int g[3];
-                if (L.corrected)
-                    grid_idx_fast(L, f3{a.x, a.y, a.z}, g);
-                else
-                    grid_idx(L, f3{a.x, a.y, a.z}, g);
-                const uint32_t h = cell_hash(g[0], g[1], g[2], L.n_paths);
-                if (!L.corrected) atomicMax(&key[h], p * nv + i + 1u);
-                atomicAdd(&count[h], 1u);
+        const unsigned long long idle = __ballot(!has);
+        const uint32_t n_idle = (uint32_t)__popcll(idle);
+        if (n_idle == 64u || (!wt.done && n_idle >= L.regen_min)) {
+            if (n_idle == 64u && wt.done) break;
+            uint32_t p = 0u;
+            if (take_items(wt, idle, p)) {
+                has = light_begin(sv, L, p, s);
+                if (!has) cnt[p] = 0u;
             }
+        }
+        if (has && !light_step<COUNT>(sv, L, cam, s, verts, splat, key, count, stk, c)) {
+            has = false;
+            cnt[s.p] = s.n;
         }
     }
     if (COUNT) flush_counts(c, counts);
@@ -309,8 +351,8 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
 
 // corrected estimator: every photon into its bucket's range
 __global__ void k_vcm_scatter(VcmLaunch L, const VcmVertex* __restrict__ verts, const uint32_t* __restrict__ cnt,
-                              const uint32_t* __restrict__ start, uint32_t* __restrict__ fill,
-                              float4* __restrict__ ppos, VcmPhotonRest* __restrict__ prest) {
+                              const uint32_t* __restrict__ start, float4* __restrict__ ppos,
+                              VcmPhotonRest* __restrict__ prest) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= L.n_paths) return;
     const uint32_t nv = (uint32_t)L.max_depth + 1u;
@@ -320,8 +362,7 @@ __global__ void k_vcm_scatter(VcmLaunch L, const VcmVertex* __restrict__ verts, 
         const uint4 f = v.f;
         int g[3];
         grid_idx_fast(L, f3{a.x, a.y, a.z}, g);
-        const uint32_t h = cell_hash(g[0], g[1], g[2], L.n_paths);
-        const uint32_t k = start[h] + atomicAdd(&fill[h], 1u);
+        const uint32_t k = start[run_bucket(g, L.n_paths)] + f.w;
         ppos[k] = a;
         VcmPhotonRest& o = prest[k];
         o.b = make_float4(-c.x, -c.y, -c.z, c.w);
@@ -484,8 +525,8 @@ LT_DEV uint32_t cell_pack(int x, int y, int z) {
 // queries the eye pass wrote.  A whole wave serves one query at a time: the
 // query and its material are wave-uniform (scalar loads and registers, and
 // the BSDF's branches on the material are uniform), the lanes load the
-// photon ranges of up to 64 of its cells at once, a wave scan lays the
-// cells' photons end to end and each lane takes every 64th photon.  A query
+// photon ranges of up to 64 of its runs of cells at once, a wave scan lays the
+// runs' photons end to end and each lane takes every 64th photon.  A query
 // over a dense caustic costs ceil(photons / 64) coalesced steps and no lane
 // waits on another lane's serial loop.  The wave's sum is added to the
 // pixel's colour with float atomics (the order of the sum is the only
@@ -505,13 +546,23 @@ constexpr int kMergeUnroll = LT_VCM_MERGE_UNROLL;
 constexpr uint32_t ring_size(uint32_t need) { return need <= 1u ? 1u : 2u * ring_size((need + 1u) / 2u); }
 constexpr uint32_t kMergeRing = ring_size(63u + 64u * (uint32_t)kMergeUnroll);
 static_assert(kMergeUnroll >= 1 && 63 + 64 * kMergeUnroll <= (int)kMergeRing, "merge ring too small");
+// A query over a caustic has up to tens of thousands of photons in its cells
+// (1,100 on average), so a wave tests at most kMergePart of a query's and lists
+// the rest, kMergePart at a time, as tasks that a second launch deals out: with
+// whole queries the waves were busy for 35 % of the pass on average, which
+// lasted as long as its heaviest wave.
+#ifndef LT_VCM_MERGE_PART
+#define LT_VCM_MERGE_PART 2048
+#endif
+constexpr uint32_t kMergePart = LT_VCM_MERGE_PART;
 // COUNT: the wave tallies the photons it tests (16 B position each), the
 // photons it merges (48 B record each) and the algorithmic bytes of its
-// queries (80-B record + 8 B of bucket range per cell) into counts[4..6].
+// queries (80-B record + 8 B of bucket range per run of cells) into counts[4..6].
 template <bool COUNT>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_VCM_MERGE_WAVES))) void k_vcm_merge(
     SceneView sv, VcmLaunch L, Grid Gr, const VcmQuery* __restrict__ queries, const uint32_t* __restrict__ n_queries,
-    float4* __restrict__ fcol, unsigned long long* __restrict__ counts) {
+    uint2* __restrict__ tasks, uint32_t* __restrict__ n_tasks, uint32_t second, float4* __restrict__ fcol,
+    unsigned long long* __restrict__ counts) {
     const uint32_t lane = threadIdx.x & 63u;
     unsigned long long n_tested = 0, n_merged = 0, n_bytes = 0;  // wave-uniform
     // photons of the wave's query that passed the distance and cell tests,
@@ -524,25 +575,44 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     float* const wd2 = s_d2[threadIdx.x / 64u];
     float* const ww = s_w[threadIdx.x / 64u];
     const uint64_t below = (1ull << lane) - 1ull;
-    const uint32_t Q = *n_queries;
     const float r2 = L.radius * L.radius;
     const float norm = 1.0f / (PI * r2 * (float)L.n_paths);
-    // Queries w, w + waves, ...: neighbouring queries (neighbouring pixels)
-    // cost alike, so the interleave balances.  Workgroups are dealt to the 8
-    // XCDs round-robin (blockIdx mod 8), each XCD with its own L2, so the
-    // wave numbering puts the waves of one XCD on consecutive queries: a
-    // round of the interleave gives each XCD one contiguous run of queries
-    // (the eye pass appends a tile's queries together, so a run is a compact
-    // image region whose cell ranges and photons its L2 then holds).  Giving
-    // each XCD one contiguous eighth of all queries instead left the XCDs
-    // unevenly loaded (3.27 against 2.51 ms per caustics frame).
-    const uint32_t wpb = blockDim.x / 64u, wib = threadIdx.x / 64u;
-    const uint32_t q_stride = gridDim.x * wpb;
-    const uint32_t q_first = (gridDim.x & 7u) == 0u
-                                 ? (blockIdx.x & 7u) * (q_stride >> 3) + (blockIdx.x >> 3) * wpb + wib
-                                 : blockIdx.x * wpb + wib;
-    const uint32_t q_end = Q;
-    for (uint32_t qi = (uint32_t)__builtin_amdgcn_readfirstlane((int)q_first); qi < q_end; qi += q_stride) {
+    // The queries lie in kQuerySegs segments, tiles s, s + kQuerySegs, ... of
+    // the image in segment s.  Workgroups are dealt to the 8 XCDs round-robin
+    // (blockIdx mod 8), each XCD with its own L2: the waves of one XCD serve 8
+    // neighbouring segments, so at any time they work on a run of 8
+    // neighbouring tiles whose bucket ranges and photons its L2 then holds;
+    // within a segment they take every n-th query (neighbouring queries cost
+    // alike, so this balances).  Giving each XCD one contiguous eighth of all
+    // queries instead left the XCDs unevenly loaded (3.27 against 2.51 ms per
+    // caustics frame).
+    const uint32_t wpb = blockDim.x / 64u, wib = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64u));
+    const uint32_t n_waves = gridDim.x * wpb;
+    uint32_t seg, q_first;
+    const uint32_t q_stride = n_waves / kQuerySegs;
+    if ((gridDim.x & 7u) == 0u) {
+        const uint32_t w = (blockIdx.x >> 3) * wpb + wib;  // this wave within its XCD
+        seg = (blockIdx.x & 7u) * (kQuerySegs / 8u) + w % (kQuerySegs / 8u);
+        q_first = w / (kQuerySegs / 8u);
+    } else {
+        const uint32_t w = blockIdx.x * wpb + wib;
+        seg = w % kQuerySegs;
+        q_first = w / kQuerySegs;
+    }
+    const uint32_t Q = q_first >= q_stride ? 0u
+                       : second            ? min(n_tasks[seg * kQueryCtrStride], kMergeTasks)
+                                           : n_queries[seg * kQueryCtrStride];
+    queries += (size_t)seg * query_seg_cap(L);
+    tasks += (size_t)seg * kMergeTasks;
+    for (uint32_t ei = (uint32_t)__builtin_amdgcn_readfirstlane((int)q_first); ei < Q; ei += q_stride) {
+        // photons [ph0, ph1) of query qi, in the order of its runs of cells
+        uint32_t qi = ei, ph0 = 0u, ph1 = kMergePart;
+        if (second) {
+            const uint2 t = tasks[ei];
+            qi = t.x;
+            ph0 = t.y * kMergePart;
+            ph1 = ph0 + kMergePart;
+        }
         const VcmQuery& qr = queries[qi];
         const float4 qa = qr.a, qb = qr.b, qc = qr.c, qd = qr.d;
         const uint4 qe = qr.e;
@@ -557,9 +627,11 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
         int lo[3], hi[3];
         grid_idx_fast(L, qpos - mk3(L.radius), lo);
         grid_idx_fast(L, qpos + mk3(L.radius), hi);
-        const int ny = hi[1] - lo[1] + 1, nz = hi[2] - lo[2] + 1;
-        const int ncells = (hi[0] - lo[0] + 1) * ny * nz;
-        if (COUNT) n_bytes += sizeof(VcmQuery) + 8ull * (unsigned long long)ncells;
+        // columns of cells along z, each in runs
+        const int r0 = lo[2] >> kRunBits, nr = (hi[2] >> kRunBits) - r0 + 1;
+        const int ny = hi[1] - lo[1] + 1;
+        const int ncells = (hi[0] - lo[0] + 1) * ny * nr;
+        if (COUNT && !second) n_bytes += sizeof(VcmQuery) + 8ull * (unsigned long long)ncells;
         f3 part = mk3(0.0f);
         uint32_t head = 0u, pend = 0u;  // wave-uniform: ring position and fill
         auto merge_slot = [&](uint32_t slot) {
@@ -571,87 +643,106 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
                           __float_as_uint(c.w), 1.0f, depth, qn, qwo, mat, side, cs, norm, r))
                 part += r;
         };
-        for (int cbase = 0; cbase < ncells; cbase += 64) {
-            const int ci = cbase + (int)lane;  // this lane's cell of the chunk: its photon range
-            uint32_t st = 0u, cnt = 0u, cpack = 0u;
-            if (ci < ncells) {
-                const int cx = lo[0] + ci / (ny * nz);
-                const int cy = lo[1] + (ci / nz) % ny;
-                const int cz = lo[2] + ci % nz;
-                cpack = cell_pack(cx, cy, cz);
-                const uint32_t h = cell_hash(cx, cy, cz, L.n_paths);
-                st = Gr.start[h];
-                cnt = Gr.start[h + 1] - st;
-            }
-            uint32_t incl = cnt;  // inclusive scan over the wave
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t v = __shfl_up(incl, (unsigned)o);
-                if ((int)lane >= o) incl += v;
-            }
-            // photon t of the chunk lies in lane j's cell at index base_j + t
-            // (modulo 2^32)
-            const uint32_t base = st - (incl - cnt);
-            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-            if (COUNT) n_tested += total;
-            // kMergeUnroll photons per lane per step: their positions are
-            // loaded together, so one memory latency covers them all
-            for (uint32_t t0 = 0; t0 < total; t0 += 64u * kMergeUnroll) {
-                uint32_t kk[kMergeUnroll], jc[kMergeUnroll];
-                bool live[kMergeUnroll];
-                float4 pa[kMergeUnroll];
-#pragma unroll
-                for (int u = 0; u < kMergeUnroll; u++) {
-                    const uint32_t t = t0 + 64u * (uint32_t)u + lane;
-                    int j = 0;  // the cell holding photon t: the first lane whose scan exceeds t
-                    for (int step = 32; step > 0; step >>= 1) {
-                        const uint32_t v = __shfl(incl, j + step - 1);
-                        if (v <= t) j += step;
-                    }
-                    j = j < 63 ? j : 63;
-                    const uint32_t bj = __shfl(base, j);
-                    jc[u] = __shfl(cpack, j);
-                    live[u] = t < total;
-                    kk[u] = live[u] ? bj + t : 0u;
+        for (;;) {
+            uint32_t seen = 0u;  // photons of the runs before this chunk
+            for (int cbase = 0; cbase < ncells; cbase += 64) {
+                const int ci = cbase + (int)lane;  // this lane's run of the chunk: its photon range
+                uint32_t st = 0u, cnt = 0u, cpack = 0u;
+                if (ci < ncells) {
+                    const int cx = lo[0] + ci / (ny * nr);
+                    const int cy = lo[1] + (ci / nr) % ny;
+                    const int run = r0 + ci % nr;
+                    cpack = cell_pack(cx, cy, run);
+                    const uint32_t h = run_base(cx, cy, run, L.n_paths);
+                    const int z0 = max(lo[2], run << kRunBits), z1 = min(hi[2], (run << kRunBits) + (1 << kRunBits) - 1);
+                    st = Gr.start[h + ((uint32_t)z0 & ((1u << kRunBits) - 1u))];
+                    cnt = Gr.start[h + ((uint32_t)z1 & ((1u << kRunBits) - 1u)) + 1u] - st;
                 }
-#pragma unroll
-                for (int u = 0; u < kMergeUnroll; u++) pa[u] = live[u] ? Gr.ppos[kk[u]] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-                for (int u = 0; u < kMergeUnroll; u++) {
-                    bool keep = false;
-                    float dist_sqr = 0.0f;
-                    if (live[u]) {
-                        const f3 ppos = {pa[u].x, pa[u].y, pa[u].z};
-                        const f3 pp = qpos - ppos;
-                        dist_sqr = dot(pp, pp);
-                        if (dist_sqr <= r2) {
-                            int g[3];
-                            grid_idx_fast(L, ppos, g);
-                            keep = cell_pack(g[0], g[1], g[2]) == jc[u];  // else another cell of the bucket
+                uint32_t incl = cnt;  // inclusive scan over the wave
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t v = __shfl_up(incl, (unsigned)o);
+                    if ((int)lane >= o) incl += v;
+                }
+                // photon t of the chunk lies in lane j's run at index base_j + t
+                // (modulo 2^32)
+                const uint32_t base = st - (incl - cnt);
+                const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+                const uint32_t t_begin = ph0 > seen ? ph0 - seen : 0u;
+                const uint32_t t_end = ph1 > seen ? min(total, ph1 - seen) : 0u;
+                seen += total;
+                if (COUNT && t_end > t_begin) n_tested += t_end - t_begin;
+                // kMergeUnroll photons per lane per step: their positions are
+                // loaded together, so one memory latency covers them all
+                for (uint32_t t0 = t_begin; t0 < t_end; t0 += 64u * kMergeUnroll) {
+                    uint32_t kk[kMergeUnroll], jc[kMergeUnroll];
+                    bool live[kMergeUnroll];
+                    float4 pa[kMergeUnroll];
+    #pragma unroll
+                    for (int u = 0; u < kMergeUnroll; u++) {
+                        const uint32_t t = t0 + 64u * (uint32_t)u + lane;
+                        int j = 0;  // the run holding photon t: the first lane whose scan exceeds t
+                        for (int step = 32; step > 0; step >>= 1) {
+                            const uint32_t v = __shfl(incl, j + step - 1);
+                            if (v <= t) j += step;
                         }
+                        j = j < 63 ? j : 63;
+                        const uint32_t bj = __shfl(base, j);
+                        jc[u] = __shfl(cpack, j);
+                        live[u] = t < t_end;
+                        kk[u] = live[u] ? bj + t : 0u;
                     }
-                    const uint64_t m = __ballot(keep);
-                    if (keep) {
-                        const uint32_t slot = (head + pend + (uint32_t)__popcll(m & below)) & (kMergeRing - 1u);
-                        wk[slot] = kk[u];
-                        wd2[slot] = dist_sqr;
-                        ww[slot] = pa[u].w;
+    #pragma unroll
+                    for (int u = 0; u < kMergeUnroll; u++) pa[u] = live[u] ? Gr.ppos[kk[u]] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    #pragma unroll
+                    for (int u = 0; u < kMergeUnroll; u++) {
+                        bool keep = false;
+                        float dist_sqr = 0.0f;
+                        if (live[u]) {
+                            const f3 ppos = {pa[u].x, pa[u].y, pa[u].z};
+                            const f3 pp = qpos - ppos;
+                            dist_sqr = dot(pp, pp);
+                            if (dist_sqr <= r2) {
+                                int g[3];
+                                grid_idx_fast(L, ppos, g);
+                                keep = cell_pack(g[0], g[1], g[2] >> kRunBits) == jc[u];  // else another run of the buckets
+                            }
+                        }
+                        const uint64_t m = __ballot(keep);
+                        if (keep) {
+                            const uint32_t slot = (head + pend + (uint32_t)__popcll(m & below)) & (kMergeRing - 1u);
+                            wk[slot] = kk[u];
+                            wd2[slot] = dist_sqr;
+                            ww[slot] = pa[u].w;
+                        }
+                        pend += (uint32_t)__popcll(m);
+                        if (COUNT) n_merged += (unsigned long long)__popcll(m);
                     }
-                    pend += (uint32_t)__popcll(m);
-                    if (COUNT) n_merged += (unsigned long long)__popcll(m);
-                }
-                while (pend >= 64u) {  // full waves of merges
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    merge_slot((head + lane) & (kMergeRing - 1u));
-                    head += 64u;
-                    pend -= 64u;
-                    // later appends reuse these slots only after every lane's reads
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    while (pend >= 64u) {  // full waves of merges
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                        merge_slot((head + lane) & (kMergeRing - 1u));
+                        head += 64u;
+                        pend -= 64u;
+                        // later appends reuse these slots only after every lane's reads
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    }
                 }
             }
+            if (second || ph0 != 0u || seen <= kMergePart) break;
+            // the rest of the query as tasks 1.. of kMergePart photons; what finds
+            // no room in the segment's list this wave does itself
+            const uint32_t parts = (seen - 1u) / kMergePart;
+            uint32_t base = 0u;
+            if (lane == 0u) base = atomicAdd(&n_tasks[seg * kQueryCtrStride], parts);
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+            const uint32_t fit = base < kMergeTasks ? min(parts, kMergeTasks - base) : 0u;
+            for (uint32_t k = lane; k < fit; k += 64u) tasks[base + k] = make_uint2(qi, k + 1u);
+            if (fit == parts) break;
+            ph0 = (fit + 1u) * kMergePart;
+            ph1 = 0xFFFFFFFFu;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -748,7 +839,7 @@ LT_DEV void eye_start(const VcmLaunch& L, const Camera& cam, uint32_t x, uint32_
 template <bool COUNT>
 LT_DEV f3 eye_wave(const SceneView& sv, const VcmLaunch& L, const Grid& G, const Camera& cam, uint32_t x, uint32_t y,
                    bool valid, VcmQuery* __restrict__ queries, uint32_t* __restrict__ n_queries,
-                   const TraceStack& stk, Ctr& c) {
+                   const TraceStack& stk, Ctr& c) {  // queries, n_queries: those of the tile's segment
     EyeState e;
     e.alive = false;
     e.col = mk3(0.0f);
@@ -867,17 +958,20 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     TraceStack stk{s_stack + threadIdx.x, spill + (size_t)gtid * (ltb::kStackTotal - ltb::kLdsStack)};
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t tiles_x = (L.width + 7) / 8, tiles_y = (L.height + 7) / 8;
-    const uint32_t n_tiles = tiles_x * tiles_y;
     const Camera cam = camera_of(L);
     Ctr c{0, 0, 0, 0};
-    for (;;) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(work, 1u);
-        t = __shfl(t, 0);
-        if (t >= n_tiles) break;
+    WaveTiles wt = wave_tiles(tiles_x * tiles_y * 64u, work);
+    while (next_tile(wt)) {
+        const uint32_t t = wt.base >> 6;
         const uint32_t x = (t % tiles_x) * 8 + (lane & 7), y = (t / tiles_x) * 8 + (lane >> 3);
+        // The queries of a tile go to the segment t mod kQuerySegs, which has a
+        // counter of its own: atomics on one counter are served one by one, 8-11
+        // ns each, and the eye pass appends about 50,000 times a frame.
+        const uint32_t seg = t % kQuerySegs;
+        VcmQuery* tq = queries ? queries + (size_t)seg * query_seg_cap(L) : nullptr;
+        uint32_t* tn = queries ? n_queries + seg * kQueryCtrStride : nullptr;
         const bool valid = x < L.width && y < L.height;
-        f3 col = eye_wave<COUNT>(sv, L, G, cam, x, y, valid, queries, n_queries, stk, c);
+        f3 col = eye_wave<COUNT>(sv, L, G, cam, x, y, valid, tq, tn, stk, c);
         if (!valid) continue;
         const size_t i = (size_t)y * L.width + x;
         if (fcol) {  // merges and the resolve follow in their own passes
@@ -964,7 +1058,6 @@ lt_status vcm_alloc(lt_context* ctx, VcmBuffers& b, uint32_t width, uint32_t hei
     LT_HIP(ctx, hipMalloc(&b.key, cells * sizeof(uint32_t)));
     LT_HIP(ctx, hipMalloc(&b.count, (cells + 1) * sizeof(uint32_t)));
     LT_HIP(ctx, hipMalloc(&b.start, (cells + 1) * sizeof(uint32_t)));
-    LT_HIP(ctx, hipMalloc(&b.fill, cells * sizeof(uint32_t)));
     LT_HIP(ctx, hipMalloc(&b.ppos, N * nv * sizeof(float4)));
     LT_HIP(ctx, hipMalloc(&b.prest, N * nv * sizeof(VcmPhotonRest)));
     LT_HIP(ctx, hipMalloc(&b.splat, N * 3 * sizeof(float)));
@@ -978,8 +1071,8 @@ lt_status vcm_alloc(lt_context* ctx, VcmBuffers& b, uint32_t width, uint32_t hei
 }
 
 void vcm_free(VcmBuffers& b) {
-    void* ptrs[] = {b.verts, b.cnt, b.key, b.count, b.start, b.fill, b.ppos, b.prest, b.scan_tmp, b.splat, b.fcol,
-                    b.queries, b.qctr};
+    void* ptrs[] = {b.verts, b.cnt, b.key, b.count, b.start, b.ppos, b.prest, b.scan_tmp, b.splat, b.fcol,
+                    b.queries, b.tasks, b.qctr};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     b = VcmBuffers{};
@@ -1005,18 +1098,22 @@ lt_status launch_vcm(lt_context* ctx, VcmBuffers& b, const VcmLaunch& L0, const 
     const bool merge_pass = L0.use_vm && L0.corrected;
     if (merge_pass && !b.queries) {
         LT_HIP(ctx, hipMalloc(&b.fcol, (size_t)b.n_paths * sizeof(float4)));
-        LT_HIP(ctx, hipMalloc(&b.queries, (size_t)b.n_paths * (size_t)b.max_depth * sizeof(VcmQuery)));
-        LT_HIP(ctx, hipMalloc(&b.qctr, 2 * sizeof(uint32_t)));
+        LT_HIP(ctx, hipMalloc(&b.queries, (size_t)kQuerySegs * query_seg_cap(L0) * sizeof(VcmQuery)));
+        LT_HIP(ctx, hipMalloc(&b.tasks, (size_t)kQuerySegs * kMergeTasks * sizeof(uint2)));
+        LT_HIP(ctx, hipMalloc(&b.qctr, 2 * kQuerySegs * kQueryCtrStride * sizeof(uint32_t)));
     }
     const uint32_t merge_blocks = ctx->num_cus * resident_blocks(reinterpret_cast<const void*>(&k_vcm_merge<false>), 0u);
     SceneView sv = make_scene_view(ctx);
     auto* cnt = (unsigned long long*)d_counts;
     if (count) fill(ctx, (uint32_t*)d_counts, 2 * kCountSlots);
     const size_t N = b.n_paths, cells = 10 * N;
-    const dim3 lgrid(light_blocks), egrid(eye_blocks), block(kTraceBlock);
+    const uint64_t tiles = (uint64_t)((L0.width + 7) / 8) * ((L0.height + 7) / 8);
+    const dim3 lgrid(work_blocks(N, light_blocks, kTraceBlock / 64)),
+        egrid(work_blocks(tiles * 64, eye_blocks, kTraceBlock / 64)), block(kTraceBlock);
     const Grid G{b.verts, b.cnt, b.key, b.count, b.start, b.ppos, b.prest};
     for (uint32_t f = 0; f < frames; f++) {
         VcmLaunch L = L0;
+        L.regen_min = ctx->tuning.regen_min ? ctx->tuning.regen_min : 4u;
         L.frame_num = frame_num + f;
         vcm_frame_words(seed, L.frame_num, &L.light_word, &L.eye_word);
         vcm_radius_grid(L.bmin, L.bmax, cfg.radius_factor, cfg.alpha, L.frame_num, &L.radius, L.grid_res);
@@ -1046,13 +1143,12 @@ lt_status launch_vcm(lt_context* ctx, VcmBuffers& b, const VcmLaunch& L0, const 
         if (L.use_vm && L.corrected) {
             LT_HIP(ctx, rocprim::exclusive_scan(b.scan_tmp, b.scan_bytes, b.count, b.start, 0u, cells + 1,
                                                 rocprim::plus<uint32_t>(), ctx->stream));
-            fill(ctx, b.fill, cells);
             hipLaunchKernelGGL(k_vcm_scatter, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, ctx->stream, L,
-                               b.verts, b.cnt, b.start, b.fill, b.ppos, b.prest);
+                               b.verts, b.cnt, b.start, b.ppos, b.prest);
         }
         float4* fcol = merge_pass ? b.fcol : nullptr;
         VcmQuery* queries = merge_pass ? b.queries : nullptr;
-        if (merge_pass) fill(ctx, b.qctr, 1);
+        if (merge_pass) fill(ctx, b.qctr, 2 * kQuerySegs * kQueryCtrStride);
         if (f == 0) phase_mark(ctx);
         if (count)
             hipLaunchKernelGGL((k_vcm_eye<true>), egrid, block, 0, ctx->stream, sv, L, G, b.splat, accum, fcol,
@@ -1062,12 +1158,15 @@ lt_status launch_vcm(lt_context* ctx, VcmBuffers& b, const VcmLaunch& L0, const 
                                queries, b.qctr, ctx->counters + 1, ctx->spill, cnt);
         if (f == 0) phase_mark(ctx);
         if (merge_pass) {
-            if (count)
-                hipLaunchKernelGGL(k_vcm_merge<true>, dim3(merge_blocks), block, 0, ctx->stream, sv, L, G, b.queries,
-                                   b.qctr, b.fcol, cnt);
-            else
-                hipLaunchKernelGGL(k_vcm_merge<false>, dim3(merge_blocks), block, 0, ctx->stream, sv, L, G, b.queries,
-                                   b.qctr, b.fcol, cnt);
+            // the queries, then the tasks that heavy ones left
+            for (uint32_t second = 0; second < 2u; second++) {
+                if (count)
+                    hipLaunchKernelGGL(k_vcm_merge<true>, dim3(merge_blocks), block, 0, ctx->stream, sv, L, G, b.queries,
+                                       b.qctr, b.tasks, b.qctr + kQuerySegs * kQueryCtrStride, second, b.fcol, cnt);
+                else
+                    hipLaunchKernelGGL(k_vcm_merge<false>, dim3(merge_blocks), block, 0, ctx->stream, sv, L, G, b.queries,
+                                       b.qctr, b.tasks, b.qctr + kQuerySegs * kQueryCtrStride, second, b.fcol, cnt);
+            }
         }
         if (f == 0) phase_mark(ctx);
         if (merge_pass) {
