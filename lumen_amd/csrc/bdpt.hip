@@ -657,8 +657,8 @@ LT_DEV f3 bdpt_connect(const SceneView& sv, const BdptLaunch& L, const VStore& v
     return col;
 }
 
-// Both kernels are persistent: each wave pulls 8x8 pixel tiles of the chunk
-// [tile0, tile0 + n_tiles) from `work`; a pixel's slot in the vertex and
+// Both kernels are persistent: each wave works through 8x8 pixel tiles of the
+// chunk [tile0, tile0 + n_tiles) (dev_work.h); a pixel's slot in the vertex and
 // record buffers is its position in the chunk.
 // The walk kernel: persistent lanes, one bounce per iteration; a lane takes
 // the next pixel of the chunk as soon as its pixel's camera subpath ends
@@ -676,7 +676,6 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     __shared__ uint32_t s_stack[ltb::kLdsWords * kTraceBlock];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     TraceStack stk{s_stack + threadIdx.x, spill + (size_t)gtid * (ltb::kStackTotal - ltb::kLdsStack)};
-    const uint32_t lane = threadIdx.x & 63u;
     const uint32_t tiles_x = (L.width + 7) / 8;
     const uint32_t n_items = n_tiles * 64u;
     const uint32_t frame_word = L.frame_dev ? (*L.frame_dev ^ L.seed) : L.frame_word;
@@ -684,40 +683,29 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     const uint32_t nv = (uint32_t)D + 1u;
     Ctr c{0, 0, 0, 0};
     WalkState w;
-    bool has = false, exhausted = false;  // exhausted is wave-uniform
+    bool has = false;
+    WaveTiles wt = wave_tiles(n_items, work);
     for (;;) {
-        if (!exhausted) {
-            const unsigned long long idle = __ballot(!has);
-            const uint32_t n_idle = (uint32_t)__popcll(idle);
-            if (n_idle >= L.regen_min || n_idle == 64u) {
-                const int leader = __ffsll((long long)idle) - 1;
-                uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(work, n_idle);
-                base = __shfl(base, leader);
-                if (base + n_idle >= n_items) exhausted = true;
-                if (!has) {
-                    const uint32_t i = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                    if (i < n_items) {
-                        const uint32_t g = tile0 + (i >> 6), q = i & 63u;
-                        const uint32_t x = (g % tiles_x) * 8 + (q & 7u), y = (g / tiles_x) * 8 + (q >> 3);
-                        if (x < L.width && y < L.height) {
-                            w.seed = {x, y, frame_word, 0u};
-                            w.slot = i;
-                            w.st = 0u;
-                            const VStore vs{verts, slots, nv, i};
-                            if (!walk_begin(sv, L, vs, hdr, w)) {
-                                w.st = 1u;  // no light subpath: n_light 0
-                                walk_begin(sv, L, vs, hdr, w);
-                            }
-                            has = true;
-                        }
+        const unsigned long long idle = __ballot(!has);
+        const uint32_t n_idle = (uint32_t)__popcll(idle);
+        if (n_idle == 64u || (!wt.done && n_idle >= L.regen_min)) {
+            if (n_idle == 64u && wt.done) break;
+            uint32_t i = 0u;
+            if (take_items(wt, idle, i)) {
+                const uint32_t g = tile0 + (i >> 6), q = i & 63u;
+                const uint32_t x = (g % tiles_x) * 8 + (q & 7u), y = (g / tiles_x) * 8 + (q >> 3);
+                if (x < L.width && y < L.height) {
+                    w.seed = {x, y, frame_word, 0u};
+                    w.slot = i;
+                    w.st = 0u;
+                    const VStore vs{verts, slots, nv, i};
+                    if (!walk_begin(sv, L, vs, hdr, w)) {
+                        w.st = 1u;  // no light subpath: n_light 0
+                        walk_begin(sv, L, vs, hdr, w);
                     }
+                    has = true;
                 }
             }
-        }
-        if (__ballot(has) == 0ull) {
-            if (exhausted) break;
-            continue;
         }
         if (has) {
             const VStore vs{verts, slots, nv, w.slot};
@@ -754,11 +742,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t tiles_x = (L.width + 7) / 8;
     Ctr c{0, 0, 0, 0};
-    for (;;) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(work, 1u);
-        t = __shfl(t, 0);
-        if (t >= n_tiles) break;
+    WaveTiles wt = wave_tiles(n_tiles * 64u, work);
+    while (next_tile(wt)) {
+        const uint32_t t = wt.base >> 6;
         const uint32_t g = tile0 + t;
         const uint32_t x = (g % tiles_x) * 8 + (lane & 7), y = (g / tiles_x) * 8 + (lane >> 3);
         if (x >= L.width || y >= L.height) continue;
@@ -868,7 +854,7 @@ lt_status launch_bdpt(lt_context* ctx, BdptBuffers& b, const BdptLaunch& L0, uin
         hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)d_counts, (size_t)(2 * kCountSlots),
                            0u);
     const uint32_t n = (uint32_t)b.pixels;
-    const dim3 wgrid(walk_blocks), cgrid(conn_blocks), block(kTraceBlock);
+    const dim3 block(kTraceBlock);
     for (uint32_t f = 0; f < frames; f++) {
         BdptLaunch L = L0;
         L.frame_word = (frame_num + f) ^ seed;
@@ -876,6 +862,8 @@ lt_status launch_bdpt(lt_context* ctx, BdptBuffers& b, const BdptLaunch& L0, uin
         L.regen_min = ctx->tuning.regen_min ? ctx->tuning.regen_min : 4u;
         for (uint32_t t0 = 0; t0 < tiles; t0 += b.chunk_tiles) {
             const uint32_t nt = tiles - t0 < b.chunk_tiles ? tiles - t0 : b.chunk_tiles;
+            const dim3 wgrid(work_blocks((uint64_t)nt * 64, walk_blocks, kTraceBlock / 64)),
+                cgrid(work_blocks((uint64_t)nt * 64, conn_blocks, kTraceBlock / 64));
             if (f == 0) phase_mark(ctx);
             hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, (size_t)2, 0u);
             if (count)

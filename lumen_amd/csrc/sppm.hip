@@ -61,9 +61,9 @@ struct SppmGrid {
 // calc_bounds.comp:16-27 from the reduced bounds
 LT_DEV SppmGrid sppm_grid(const SppmBounds& b) {
     SppmGrid g;
-    g.mn = {ord_dec(b.mn[0]), ord_dec(b.mn[1]), ord_dec(b.mn[2])};
-    g.mx = {ord_dec(b.mx[0]), ord_dec(b.mx[1]), ord_dec(b.mx[2])};
-    const float max_r = ord_dec(b.max_r);
+    g.mn = {ord_dec(b.mn[0].v), ord_dec(b.mn[1].v), ord_dec(b.mn[2].v)};
+    g.mx = {ord_dec(b.mx[0].v), ord_dec(b.mx[1].v), ord_dec(b.mx[2].v)};
+    const float max_r = ord_dec(b.max_r.v);
     const f3 ext = g.mx - g.mn;
     const float max_comp = fmaxf(ext.x, fmaxf(ext.y, ext.z));
     const int base = (int)(max_comp / max_r);
@@ -114,96 +114,112 @@ __global__ void k_sppm_clear(uint32_t* key, uint32_t* count, size_t cells, float
         for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < state_words; i += stride) state[i] = 0.0f;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         for (int k = 0; k < 3; k++) {
-            bounds->mn[k] = 0xFFFFFFFFu;  // above every encoded float
-            bounds->mx[k] = 0u;
+            bounds->mn[k].v = 0xFFFFFFFFu;  // above every encoded float
+            bounds->mx[k].v = 0u;
         }
-        bounds->max_r = 0u;
+        bounds->max_r.v = 0u;
     }
 }
 
-// sppm_eye.rgen:42-128 for pixel (x, y), state index q = y * W + x
-template <bool COUNT>
-LT_DEV void eye_path(const SceneView& sv, const SppmLaunch& L, uint32_t x, uint32_t y, float* st,
-                     const TraceStack& stk, Ctr& c) {
+// An eye path between two bounces (sppm_eye.rgen:42-128); the recorded point
+// goes straight to the pixel's planes.
+struct EyeState {
+    f3 origin, direction, thr, col;
+    uint32_t xy, rng;  // x | y << 16, RNG counter
+    int depth;
+    bool specular, recorded;
+};
+
+LT_DEV void eye_begin(const SppmLaunch& L, uint32_t x, uint32_t y, const float* st, EyeState& e) {
     const uint32_t n = L.n_px, q = y * L.width + x;
-    RNG seed = {x, y, L.word, 0u};
     const float dx = ((float)x + 0.5f) / (float)L.width * 2.0f - 1.0f;
     const float dy = ((float)y + 0.5f) / (float)L.height * 2.0f - 1.0f;
     const f4 o4 = mul4(L.inv_view, f4{0.0f, 0.0f, 0.0f, 1.0f});
     const f4 tg = mul4(L.inv_projection, f4{dx, dy, 1.0f, 1.0f});
     const f3 tn = normalize(mk3(tg.x, tg.y, tg.z));
     const f4 d4 = mul4(L.inv_view, f4{tn.x, tn.y, tn.z, 0.0f});
-    f3 origin = {o4.x, o4.y, o4.z}, direction = {d4.x, d4.y, d4.z};
-    f3 thr = mk3(1.0f);
-    f3 col = {ld_plane(st, n, kSpColx, q), ld_plane(st, n, kSpColy, q), ld_plane(st, n, kSpColz, q)};
-    bool specular = false, recorded = false;
+    e.origin = {o4.x, o4.y, o4.z};
+    e.direction = {d4.x, d4.y, d4.z};
+    e.thr = mk3(1.0f);
+    e.col = {ld_plane(st, n, kSpColx, q), ld_plane(st, n, kSpColy, q), ld_plane(st, n, kSpColz, q)};
+    e.xy = x | (y << 16);
+    e.rng = 0u;
+    e.depth = 0;
+    e.specular = e.recorded = false;
+}
+
+// One bounce; false once the path has ended.
+template <bool COUNT>
+LT_DEV bool eye_step(const SceneView& sv, const SppmLaunch& L, EyeState& e, float* st, const TraceStack& stk, Ctr& c) {
+    const uint32_t n = L.n_px, x = e.xy & 0xFFFFu, y = e.xy >> 16, q = y * L.width + x;
+    const int depth = e.depth++;
     Payload hp;
-    for (int depth = 0;; depth++) {
-        trace_closest<COUNT>(sv, origin, direction, stk, hp, c);
-        if (!hp.valid) {
-            col += thr * ld3(L.sky_col);
-            break;
-        }
-        if (depth >= L.max_depth - 1) break;
-        const Mat mat = load_material(sv, hp.material_idx, hp.uv);
-        if (depth == 0 || (specular && !recorded)) col += thr * mat.emissive;
-        const f3 wo = -direction;
-        f3 n_s = hp.n_s, n_g = hp.n_g;
-        bool side = true;
-        if (dot(hp.n_g, wo) < 0.0f) n_g = -n_g;
-        if (dot(n_g, hp.n_s) < 0.0f) {
-            n_s = -n_s;
-            side = false;
-        }
-        const f3 pos = hp.pos;
-        origin = offset_ray(pos, n_g);
-        specular = is_specular(mat);
-        if (!recorded && !specular) {  // sppm_eye.rgen:91-96: Path's NEE / (1 / light_triangle_count)
-            NeeRays nee;
-            nee_sample(sv, seed, mat, hp, side, n_s, wo, thr, LT_NEE_REFERENCE, nee);
-            col += nee_trace<COUNT>(sv, nee, stk, c);
-        }
-        if (!recorded && (mat.bsdf_type & LT_BSDF_DIFFUSE) != 0u) {  // sppm_eye.rgen:99-110
-            recorded = true;
-            st_plane(st, n, kSpWox, q, wo.x);
-            st_plane(st, n, kSpWoy, q, wo.y);
-            st_plane(st, n, kSpWoz, q, wo.z);
-            st_plane(st, n, kSpPx, q, pos.x);
-            st_plane(st, n, kSpPy, q, pos.y);
-            st_plane(st, n, kSpPz, q, pos.z);
-            st_plane(st, n, kSpMat, q, __uint_as_float(hp.material_idx));
-            st_plane(st, n, kSpU, q, hp.uv.x);
-            st_plane(st, n, kSpV, q, hp.uv.y);
-            st_plane(st, n, kSpThrx, q, thr.x);
-            st_plane(st, n, kSpThry, q, thr.y);
-            st_plane(st, n, kSpThrz, q, thr.z);
-            st_plane(st, n, kSpNx, q, n_s.x);
-            st_plane(st, n, kSpNy, q, n_s.y);
-            st_plane(st, n, kSpNz, q, n_s.z);
-            st_plane(st, n, kSpPathLen, q, __int_as_float(depth));
-            st_plane(st, n, kSpSide, q, __uint_as_float(side ? 1u : 0u));
-        }
-        float pdf, cos_theta;
-        const float r0 = rnd(seed), r1 = rnd(seed), r2 = rnd(seed);
-        const f3 f = sample_bsdf(n_s, wo, mat, 1u, side, direction, pdf, cos_theta, r0, r1, r2);
-        if (pdf < 1e-20f || dot(f, f) < 1e-20f) break;
-        thr *= f * fabsf(cos_theta) / pdf;
-        if (depth > RR_MIN_DEPTH) {  // no 0.95 cap in the eye pass (sppm_eye.rgen:118-124)
-            const float rr_prob = luminance(thr);
-            if (rr_prob < rnd(seed)) break;
-            thr /= rr_prob;
-        }
+    trace_closest<COUNT>(sv, e.origin, e.direction, stk, hp, c);
+    if (!hp.valid) {
+        e.col += e.thr * ld3(L.sky_col);
+        return false;
     }
-    st_plane(st, n, kSpColx, q, col.x);
-    st_plane(st, n, kSpColy, q, col.y);
-    st_plane(st, n, kSpColz, q, col.z);
-    if (L.frame_num == 0u) st_plane(st, n, kSpRadius, q, L.base_radius);
+    if (depth >= L.max_depth - 1) return false;
+    RNG seed = {x, y, L.word, e.rng};
+    const Mat mat = load_material(sv, hp.material_idx, hp.uv);
+    if (depth == 0 || (e.specular && !e.recorded)) e.col += e.thr * mat.emissive;
+    const f3 wo = -e.direction;
+    f3 n_s = hp.n_s, n_g = hp.n_g;
+    bool side = true;
+    if (dot(hp.n_g, wo) < 0.0f) n_g = -n_g;
+    if (dot(n_g, hp.n_s) < 0.0f) {
+        n_s = -n_s;
+        side = false;
+    }
+    const f3 pos = hp.pos;
+    e.origin = offset_ray(pos, n_g);
+    e.specular = is_specular(mat);
+    if (!e.recorded && !e.specular) {  // sppm_eye.rgen:91-96: Path's NEE / (1 / light_triangle_count)
+        NeeRays nee;
+        nee_sample(sv, seed, mat, hp, side, n_s, wo, e.thr, LT_NEE_REFERENCE, nee);
+        e.col += nee_trace<COUNT>(sv, nee, stk, c);
+    }
+    if (!e.recorded && (mat.bsdf_type & LT_BSDF_DIFFUSE) != 0u) {  // sppm_eye.rgen:99-110
+        e.recorded = true;
+        st_plane(st, n, kSpWox, q, wo.x);
+        st_plane(st, n, kSpWoy, q, wo.y);
+        st_plane(st, n, kSpWoz, q, wo.z);
+        st_plane(st, n, kSpPx, q, pos.x);
+        st_plane(st, n, kSpPy, q, pos.y);
+        st_plane(st, n, kSpPz, q, pos.z);
+        st_plane(st, n, kSpMat, q, __uint_as_float(hp.material_idx));
+        st_plane(st, n, kSpU, q, hp.uv.x);
+        st_plane(st, n, kSpV, q, hp.uv.y);
+        st_plane(st, n, kSpThrx, q, e.thr.x);
+        st_plane(st, n, kSpThry, q, e.thr.y);
+        st_plane(st, n, kSpThrz, q, e.thr.z);
+        st_plane(st, n, kSpNx, q, n_s.x);
+        st_plane(st, n, kSpNy, q, n_s.y);
+        st_plane(st, n, kSpNz, q, n_s.z);
+        st_plane(st, n, kSpPathLen, q, __int_as_float(depth));
+        st_plane(st, n, kSpSide, q, __uint_as_float(side ? 1u : 0u));
+    }
+    float pdf, cos_theta;
+    const float r0 = rnd(seed), r1 = rnd(seed), r2 = rnd(seed);
+    e.rng = seed.w;
+    const f3 f = sample_bsdf(n_s, wo, mat, 1u, side, e.direction, pdf, cos_theta, r0, r1, r2);
+    if (pdf < 1e-20f || dot(f, f) < 1e-20f) return false;
+    e.thr *= f * fabsf(cos_theta) / pdf;
+    if (depth > RR_MIN_DEPTH) {  // no 0.95 cap in the eye pass (sppm_eye.rgen:118-124)
+        const float rr_prob = luminance(e.thr);
+        const float r = rnd(seed);
+        e.rng = seed.w;
+        if (rr_prob < r) return false;
+        e.thr /= rr_prob;
+    }
+    return true;
 }
 
 #ifndef LT_SPPM_EYE_WAVES
 #define LT_SPPM_EYE_WAVES 4
 #endif
-// persistent waves pulling 8x8 pixel tiles
+// persistent lanes over 8x8 pixel tiles: one bounce per iteration, a lane takes
+// the next pixel as soon as its path ends
 template <bool COUNT>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_SPPM_EYE_WAVES))) void k_sppm_eye(
     SceneView sv, SppmLaunch L, float* __restrict__ st, uint32_t* __restrict__ work, uint32_t* __restrict__ spill,
@@ -211,16 +227,34 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     __shared__ uint32_t s_stack[ltb::kLdsWords * kTraceBlock];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     TraceStack stk{s_stack + threadIdx.x, spill + (size_t)gtid * (ltb::kStackTotal - ltb::kLdsStack)};
-    const uint32_t lane = threadIdx.x & 63u;
     const uint32_t tiles_x = (L.width + 7) / 8, n_tiles = tiles_x * ((L.height + 7) / 8);
     Ctr c{0, 0, 0, 0};
+    EyeState e;
+    bool has = false;
+    WaveTiles wt = wave_tiles(n_tiles * 64u, work);
     for (;;) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(work, 1u);
-        t = __shfl(t, 0);
-        if (t >= n_tiles) break;
-        const uint32_t x = (t % tiles_x) * 8 + (lane & 7u), y = (t / tiles_x) * 8 + (lane >> 3);
-        if (x < L.width && y < L.height) eye_path<COUNT>(sv, L, x, y, st, stk, c);
+        const unsigned long long idle = __ballot(!has);
+        const uint32_t n_idle = (uint32_t)__popcll(idle);
+        if (n_idle == 64u || (!wt.done && n_idle >= L.regen_min)) {
+            if (n_idle == 64u && wt.done) break;
+            uint32_t i = 0u;
+            if (take_items(wt, idle, i)) {
+                const uint32_t t = i >> 6, w = i & 63u;
+                const uint32_t x = (t % tiles_x) * 8 + (w & 7u), y = (t / tiles_x) * 8 + (w >> 3);
+                if (x < L.width && y < L.height) {
+                    eye_begin(L, x, y, st, e);
+                    has = true;
+                }
+            }
+        }
+        if (has && !eye_step<COUNT>(sv, L, e, st, stk, c)) {
+            has = false;
+            const uint32_t n = L.n_px, q = (e.xy >> 16) * L.width + (e.xy & 0xFFFFu);
+            st_plane(st, n, kSpColx, q, e.col.x);
+            st_plane(st, n, kSpColy, q, e.col.y);
+            st_plane(st, n, kSpColz, q, e.col.z);
+            if (L.frame_num == 0u) st_plane(st, n, kSpRadius, q, L.base_radius);
+        }
     }
     if (COUNT) flush_counts(c, counts);
 }
@@ -269,18 +303,22 @@ __global__ __launch_bounds__(256) void k_sppm_bounds(const float* __restrict__ s
             mr = fmaxf(mr, red[v][6]);
         }
         for (int k = 0; k < 3; k++) {
-            atomicMin(&b->mn[k], ord_enc(lo[k]));
-            atomicMax(&b->mx[k], ord_enc(hi[k]));
+            atomicMin(&b->mn[k].v, ord_enc(lo[k]));
+            atomicMax(&b->mx[k].v, ord_enc(hi[k]));
         }
-        atomicMax(&b->max_r, ord_enc(mr));
+        atomicMax(&b->max_r.v, ord_enc(mr));
     }
 }
 
-// sppm_light.rgen:43-114 for the light path of pixel slot q (x = q % W, y = q / W)
-template <bool COUNT>
-LT_DEV void light_path(const SceneView& sv, const SppmLaunch& L, const SppmGrid& g, uint32_t q,
-                       SppmPhoton* __restrict__ photons, uint32_t* __restrict__ key, uint32_t* __restrict__ count,
-                       const TraceStack& stk, Ctr& c) {
+// A light path between two bounces (sppm_light.rgen:43-114), of pixel slot q
+// (x = q % W, y = q / W).
+struct LightState {
+    f3 pos, wi, thr;
+    uint32_t q, rng;
+    int depth;
+};
+
+LT_DEV void light_begin(const SceneView& sv, const SppmLaunch& L, uint32_t q, LightState& s) {
     RNG seed = {q % L.width, q / L.width, L.word, 0u};
     f4 rp;
     rp.x = rnd(seed);
@@ -290,54 +328,68 @@ LT_DEV void light_path(const SceneView& sv, const SppmLaunch& L, const SppmGrid&
     const float rd0 = rnd(seed), rd1 = rnd(seed);
     float cos_theta, pdf_pos, pdf_dir;
     uint32_t flags, li;
-    f3 pos, wi, n;
-    const f3 Le = sample_light_Le(sv, rp, rd0, rd1, cos_theta, flags, li, pos, wi, n, pdf_pos, pdf_dir);
-    const float abs_cos = fabsf(dot(n, wi));
-    f3 thr = (abs_cos == 0.0f || pdf_dir <= 0.0f) ? mk3(0.0f) : Le * abs_cos / (pdf_dir * pdf_pos);
-    for (int depth = 0; depth < L.max_depth; depth++) {
-        Payload pl;
-        if (COUNT) c.closest++;
-        HitRec h;
-        if (!trace_bvh<false, COUNT>(sv, pos, wi, SPPM_TMIN, SPPM_TMAX, h, stk, c.nodes, c.tris)) break;
-        fill_payload(sv, h.inst, h.prim, h.u, h.v, pl);
-        const f3 wo = -wi;
-        f3 n_s = pl.n_s, n_g = pl.n_g;
-        bool side = true;
-        if (dot(pl.n_g, wo) < 0.0f) n_g = -n_g;
-        if (dot(n_g, pl.n_s) < 0.0f) {
-            n_s = -n_s;
-            side = false;
-        }
-        const Mat mat = load_material(sv, pl.material_idx, pl.uv);
-        if (depth > 0) {  // sppm_light.rgen:81-94: the first bounce is not stored
-            int gi[3];
-            sppm_cell(g, pl.pos, gi);
-            const uint32_t hb = sppm_hash(gi[0], gi[1], gi[2], L.n_px);
-            const uint32_t ref = q * (uint32_t)L.max_depth + (uint32_t)depth;
-            SppmPhoton& ph = photons[ref];
-            ph.a = make_float4(pl.pos.x, pl.pos.y, pl.pos.z, __uint_as_float((uint32_t)depth + 1u));
-            ph.b = make_float4(-wi.x, -wi.y, -wi.z, thr.x);
-            ph.c = make_float4(thr.y, thr.z, 0.0f, 0.0f);
-            atomicMax(&key[hb], ref + 1u);
-            atomicAdd(&count[hb], 1u);
-        }
-        pos = offset_ray(pl.pos, n_g);
-        float pdf, cos_t;
-        const float r0 = rnd(seed), r1 = rnd(seed), r2 = rnd(seed);
-        const f3 f = sample_bsdf(n_s, wo, mat, 0u, side, wi, pdf, cos_t, r0, r1, r2);
-        thr *= f * fabsf(cos_t) / pdf;
-        if ((f.x == 0.0f && f.y == 0.0f && f.z == 0.0f) || pdf == 0.0f) break;
-        if (depth > RR_MIN_DEPTH) {
-            const float rr_prob = fminf(0.95f, luminance(thr));
-            if (rr_prob < rnd(seed)) break;
-            thr /= rr_prob;
-        }
+    f3 n;
+    const f3 Le = sample_light_Le(sv, rp, rd0, rd1, cos_theta, flags, li, s.pos, s.wi, n, pdf_pos, pdf_dir);
+    const float abs_cos = fabsf(dot(n, s.wi));
+    s.thr = (abs_cos == 0.0f || pdf_dir <= 0.0f) ? mk3(0.0f) : Le * abs_cos / (pdf_dir * pdf_pos);
+    s.q = q;
+    s.rng = seed.w;
+    s.depth = 0;
+}
+
+// One bounce; false once the path has ended.
+template <bool COUNT>
+LT_DEV bool light_step(const SceneView& sv, const SppmLaunch& L, const SppmGrid& g, LightState& s,
+                       SppmPhoton* __restrict__ photons, uint32_t* __restrict__ key, uint32_t* __restrict__ count,
+                       const TraceStack& stk, Ctr& c) {
+    const int depth = s.depth++;
+    Payload pl;
+    if (COUNT) c.closest++;
+    HitRec h;
+    if (!trace_bvh<false, COUNT>(sv, s.pos, s.wi, SPPM_TMIN, SPPM_TMAX, h, stk, c.nodes, c.tris)) return false;
+    fill_payload(sv, h.inst, h.prim, h.u, h.v, pl);
+    const f3 wo = -s.wi;
+    f3 n_s = pl.n_s, n_g = pl.n_g;
+    bool side = true;
+    if (dot(pl.n_g, wo) < 0.0f) n_g = -n_g;
+    if (dot(n_g, pl.n_s) < 0.0f) {
+        n_s = -n_s;
+        side = false;
     }
+    const Mat mat = load_material(sv, pl.material_idx, pl.uv);
+    if (depth > 0) {  // sppm_light.rgen:81-94: the first bounce is not stored
+        int gi[3];
+        sppm_cell(g, pl.pos, gi);
+        const uint32_t hb = sppm_hash(gi[0], gi[1], gi[2], L.n_px);
+        const uint32_t ref = s.q * (uint32_t)L.max_depth + (uint32_t)depth;
+        SppmPhoton& ph = photons[ref];
+        ph.a = make_float4(pl.pos.x, pl.pos.y, pl.pos.z, __uint_as_float((uint32_t)depth + 1u));
+        ph.b = make_float4(-s.wi.x, -s.wi.y, -s.wi.z, s.thr.x);
+        ph.c = make_float4(s.thr.y, s.thr.z, 0.0f, 0.0f);
+        atomicMax(&key[hb], ref + 1u);
+        atomicAdd(&count[hb], 1u);
+    }
+    s.pos = offset_ray(pl.pos, n_g);
+    float pdf, cos_t;
+    RNG seed = {s.q % L.width, s.q / L.width, L.word, s.rng};
+    const float r0 = rnd(seed), r1 = rnd(seed), r2 = rnd(seed);
+    const f3 f = sample_bsdf(n_s, wo, mat, 0u, side, s.wi, pdf, cos_t, r0, r1, r2);
+    s.thr *= f * fabsf(cos_t) / pdf;
+    if ((f.x == 0.0f && f.y == 0.0f && f.z == 0.0f) || pdf == 0.0f) return false;
+    if (depth > RR_MIN_DEPTH) {
+        const float rr_prob = fminf(0.95f, luminance(s.thr));
+        if (rr_prob < rnd(seed)) return false;
+        s.thr /= rr_prob;
+    }
+    s.rng = seed.w;
+    return depth + 1 < L.max_depth;
 }
 
 #ifndef LT_SPPM_LIGHT_WAVES
 #define LT_SPPM_LIGHT_WAVES 4
 #endif
+// persistent lanes: one bounce per iteration, a lane takes the next path as
+// soon as its own ends
 template <bool COUNT>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_SPPM_LIGHT_WAVES))) void k_sppm_light(
     SceneView sv, SppmLaunch L, const SppmBounds* __restrict__ bounds, SppmPhoton* __restrict__ photons,
@@ -346,17 +398,23 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     __shared__ uint32_t s_stack[ltb::kLdsWords * kTraceBlock];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     TraceStack stk{s_stack + threadIdx.x, spill + (size_t)gtid * (ltb::kStackTotal - ltb::kLdsStack)};
-    const uint32_t lane = threadIdx.x & 63u;
     const SppmGrid g = sppm_grid(*bounds);
-    const uint32_t chunks = (L.n_px + 63u) / 64u;
     Ctr c{0, 0, 0, 0};
+    LightState s;
+    bool has = false;
+    WaveTiles wt = wave_tiles(L.n_px, work);
     for (;;) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(work, 1u);
-        t = __shfl(t, 0);
-        if (t >= chunks) break;
-        const uint32_t q = t * 64u + lane;
-        if (q < L.n_px) light_path<COUNT>(sv, L, g, q, photons, key, count, stk, c);
+        const unsigned long long idle = __ballot(!has);
+        const uint32_t n_idle = (uint32_t)__popcll(idle);
+        if (n_idle == 64u || (!wt.done && n_idle >= L.regen_min)) {
+            if (n_idle == 64u && wt.done) break;
+            uint32_t q = 0u;
+            if (take_items(wt, idle, q)) {
+                light_begin(sv, L, q, s);
+                has = true;
+            }
+        }
+        if (has && !light_step<COUNT>(sv, L, g, s, photons, key, count, stk, c)) has = false;
     }
     if (COUNT) flush_counts(c, counts);
 }
@@ -539,29 +597,33 @@ lt_status launch_sppm(lt_context* ctx, SppmBuffers& b, const SppmLaunch& L0, uin
     const size_t N = b.n_px, cells = 10 * N;
     const unsigned clear_blocks = (unsigned)std::min<size_t>((cells + 255) / 256, 8192);
     const unsigned px_blocks = (unsigned)((N + 255) / 256);
+    const uint64_t tiles = (uint64_t)((L0.width + 7) / 8) * ((L0.height + 7) / 8);
+    const dim3 egrid(work_blocks(tiles * 64, eye_blocks, kTraceBlock / 64)),
+        lgrid(work_blocks(N, light_blocks, kTraceBlock / 64));
     for (uint32_t f = 0; f < frames; f++) {
         SppmLaunch L = L0;
         L.frame_num = frame_num + f;
         L.word = sppm_frame_word(seed, L.frame_num);
+        L.regen_min = ctx->tuning.regen_min ? ctx->tuning.regen_min : 4u;
         if (f == 0) phase_mark(ctx);
         hipLaunchKernelGGL(k_sppm_clear, dim3(clear_blocks), dim3(256), 0, ctx->stream, b.key, b.count, cells,
                            b.state, N * kSpPlanes, L.frame_num == 0u ? 1 : 0, b.bounds);
         hipLaunchKernelGGL(k_sppm_fill, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 2u);
         if (count)
-            hipLaunchKernelGGL((k_sppm_eye<true>), dim3(eye_blocks), dim3(kTraceBlock), 0, ctx->stream, sv, L,
+            hipLaunchKernelGGL((k_sppm_eye<true>), egrid, dim3(kTraceBlock), 0, ctx->stream, sv, L,
                                b.state, ctx->counters, ctx->spill, cnt);
         else
-            hipLaunchKernelGGL((k_sppm_eye<false>), dim3(eye_blocks), dim3(kTraceBlock), 0, ctx->stream, sv, L,
+            hipLaunchKernelGGL((k_sppm_eye<false>), egrid, dim3(kTraceBlock), 0, ctx->stream, sv, L,
                                b.state, ctx->counters, ctx->spill, cnt);
         if (f == 0) phase_mark(ctx);
         hipLaunchKernelGGL(k_sppm_bounds, dim3((unsigned)std::min<size_t>((N + 255) / 256, 4u * ctx->num_cus)),
                            dim3(256), 0, ctx->stream, b.state, (uint32_t)N, b.bounds);
         if (f == 0) phase_mark(ctx);
         if (count)
-            hipLaunchKernelGGL((k_sppm_light<true>), dim3(light_blocks), dim3(kTraceBlock), 0, ctx->stream, sv, L,
+            hipLaunchKernelGGL((k_sppm_light<true>), lgrid, dim3(kTraceBlock), 0, ctx->stream, sv, L,
                                b.bounds, b.photons, b.key, b.count, ctx->counters + 1, ctx->spill, cnt);
         else
-            hipLaunchKernelGGL((k_sppm_light<false>), dim3(light_blocks), dim3(kTraceBlock), 0, ctx->stream, sv, L,
+            hipLaunchKernelGGL((k_sppm_light<false>), lgrid, dim3(kTraceBlock), 0, ctx->stream, sv, L,
                                b.bounds, b.photons, b.key, b.count, ctx->counters + 1, ctx->spill, cnt);
         if (f == 0) phase_mark(ctx);
         if (count)
