@@ -217,29 +217,35 @@ LT_DEV bool walk_step(const SceneView& sv, const VStore& vs, int max_depth, Walk
     return true;
 }
 
-// The MIS prefix sums of the unmodified vertices (see the file comment).
+// The MIS prefix sums of the unmodified vertices of subpath `sub` (see the
+// file comment), and each vertex's predecessor delta flag as bit 2 of its bits:
 //   camera: P_0 = 0, P_k = r_k (c_k + P_{k-1}), c_k = !delta_k && !delta_{k-1}
 //   light:  Q_{-1} = 0, Q_k = r_k (c_k + Q_{k-1}), c_k = !delta_k && !dprev_k,
 //           dprev_0 = the light is a delta light
-LT_DEV void mis_prefixes(const VStore& vs, int n_light, int n_cam, bool light_is_delta, bool power) {
+// The next vertex's fields are loaded before this one's are stored.
+LT_DEV void mis_prefixes(const VStore& vs, int sub, int n, bool light_is_delta, bool power) {
+    if (n <= 0) return;
     float P = 0.0f;
-    uint32_t dprev = vs.getu(1, 0, F_BITS) & 1u;
-    vs.put(1, 0, F_PRE, 0.0f);
-    for (int k = 1; k < n_cam; k++) {
-        const uint32_t d = vs.getu(1, k, F_BITS) & 1u;
-        const float r = mis_term(remap0(vs.get(1, k, F_PREV)) / remap0(vs.get(1, k, F_PFWD)), power);
-        P = r * (((d == 0u && dprev == 0u) ? 1.0f : 0.0f) + P);
-        vs.put(1, k, F_PRE, P);
+    uint32_t dprev = light_is_delta ? 1u : 0u;
+    uint32_t bits = vs.getu(sub, 0, F_BITS);
+    float rev = vs.get(sub, 0, F_PREV), fwd = vs.get(sub, 0, F_PFWD);
+    for (int k = 0; k < n; k++) {
+        const int nx = k + 1 < n ? k + 1 : k;
+        const uint32_t bits_n = vs.getu(sub, nx, F_BITS);
+        const float rev_n = vs.get(sub, nx, F_PREV), fwd_n = vs.get(sub, nx, F_PFWD);
+        const uint32_t d = bits & 1u;
+        if (sub == 1 && k == 0) {
+            P = 0.0f;
+        } else {
+            const float r = mis_term(remap0(rev) / remap0(fwd), power);
+            P = r * (((d == 0u && dprev == 0u) ? 1.0f : 0.0f) + P);
+            if (dprev) vs.putu(sub, k, F_BITS, bits | 4u);
+        }
+        vs.put(sub, k, F_PRE, P);
         dprev = d;
-    }
-    float Q = 0.0f;
-    bool dp = light_is_delta;
-    for (int k = 0; k < n_light; k++) {
-        const uint32_t d = vs.getu(0, k, F_BITS) & 1u;
-        const float r = mis_term(remap0(vs.get(0, k, F_PREV)) / remap0(vs.get(0, k, F_PFWD)), power);
-        Q = r * (((d == 0u && !dp) ? 1.0f : 0.0f) + Q);
-        vs.put(0, k, F_PRE, Q);
-        dp = d == 1u;
+        bits = bits_n;
+        rev = rev_n;
+        fwd = fwd_n;
     }
 }
 
@@ -443,22 +449,31 @@ LT_DEV bool walk_begin(const SceneView& sv, const BdptLaunch& L, const VStore& v
     return true;
 }
 
-// After both subpaths: the predecessor's delta flag as bit 2 of each vertex,
-// the MIS prefixes, and the rest of the pixel record (subpath lengths, the
-// RNG counter) for the connection kernel.
-LT_DEV void walk_finish(const BdptLaunch& L, const VStore& vs, uint32_t* __restrict__ hdr, const WalkState& w) {
-    const int n_light = w.n_light(), n_cam = w.b() + 1;
+// After both subpaths: the rest of the pixel record (subpath lengths, the RNG
+// counter) for the prefix and connection kernels.
+LT_DEV void walk_finish(const VStore& vs, uint32_t* __restrict__ hdr, const WalkState& w) {
     const size_t S = vs.slots;
-    const bool delta0 = light_delta(hdr[H_FLAGS * S + vs.slot]);
-    for (int k = 1; k < n_cam; k++)
-        vs.putu(1, k, F_BITS, vs.getu(1, k, F_BITS) | ((vs.getu(1, k - 1, F_BITS) & 1u) << 2));
-    for (int k = 0; k < n_light; k++) {
-        const uint32_t dp = k > 0 ? (vs.getu(0, k - 1, F_BITS) & 1u) : (delta0 ? 1u : 0u);
-        vs.putu(0, k, F_BITS, vs.getu(0, k, F_BITS) | (dp << 2));
-    }
-    mis_prefixes(vs, n_light, n_cam, delta0, L.power != 0u);
-    hdr[H_COUNTS * S + vs.slot] = (uint32_t)n_light | ((uint32_t)n_cam << 8);
+    hdr[H_COUNTS * S + vs.slot] = (uint32_t)w.n_light() | ((uint32_t)(w.b() + 1) << 8);
     hdr[H_SEEDW * S + vs.slot] = w.seed.w;
+}
+
+// The MIS prefixes of the chunk's pixels, a thread per subpath.  In the walk
+// kernel, where a lane finished its pixel whenever its path ended, this ran for
+// a few lanes of a wave at a time over up to 18 vertices, one memory latency
+// after another, nearly every iteration; here neighbouring lanes read and write
+// neighbouring words (HBM bound: 20 B per vertex).
+__global__ __launch_bounds__(256) void k_bdpt_prefix(BdptLaunch L, float* __restrict__ verts,
+                                                     const uint32_t* __restrict__ hdr, uint32_t slots, uint32_t tile0,
+                                                     uint32_t n_tiles) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_tiles * 64u) return;
+    const int sub = (int)blockIdx.y;
+    const uint32_t tiles_x = (L.width + 7) / 8, g = tile0 + (i >> 6), q = i & 63u;
+    if ((g % tiles_x) * 8 + (q & 7u) >= L.width || (g / tiles_x) * 8 + (q >> 3) >= L.height) return;
+    const VStore vs{verts, slots, (uint32_t)L.max_depth + 1u, i};
+    const uint32_t counts = hdr[H_COUNTS * (size_t)slots + i];
+    const int n = sub == 0 ? (int)(counts & 0xFFu) : (int)(counts >> 8);
+    mis_prefixes(vs, sub, n, sub == 0 && light_delta(hdr[H_FLAGS * (size_t)slots + i]), L.power != 0u);
 }
 
 // Connection kernel body for pixel (x, y): every (s, t) strategy of
@@ -716,7 +731,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
                     w.st = 1u | ((uint32_t)(w.b() + 1) << 16);
                     walk_begin(sv, L, vs, hdr, w);
                 } else {
-                    walk_finish(L, vs, hdr, w);
+                    walk_finish(vs, hdr, w);
                     has = false;
                 }
             }
@@ -872,6 +887,8 @@ lt_status launch_bdpt(lt_context* ctx, BdptBuffers& b, const BdptLaunch& L0, uin
             else
                 hipLaunchKernelGGL((k_bdpt_walk<false>), wgrid, block, 0, ctx->stream, sv, L, b.verts, b.hdr, b.slots,
                                    t0, nt, ctx->counters, ctx->spill, cnt);
+            hipLaunchKernelGGL(k_bdpt_prefix, dim3((nt * 64 + 255) / 256, 2), dim3(256), 0, ctx->stream, L, b.verts,
+                               b.hdr, b.slots, t0, nt);
             if (f == 0) phase_mark(ctx);
             if (count)
                 hipLaunchKernelGGL((k_bdpt_connect<true>), cgrid, block, 0, ctx->stream, sv, L, b.verts, b.hdr,
