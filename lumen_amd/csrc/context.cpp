@@ -180,7 +180,7 @@ lt_status lt_context_destroy(lt_context* ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     free_scene(ctx->scene);
     free_bvh(ctx->bvh);
-    void* ptrs[] = {ctx->spill, ctx->counters, ctx->ray_buf, ctx->hit_buf, ctx->count_buf};
+    void* ptrs[] = {ctx->spill, ctx->build_ws, ctx->counters, ctx->ray_buf, ctx->hit_buf, ctx->count_buf};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (hipEvent_t& e : ctx->phase_ev)

@@ -100,6 +100,9 @@ struct lt_context {
     // traversal stack spill (kStackTotal - kLdsStack entries per resident thread)
     uint32_t* spill = nullptr;
     size_t spill_threads = 0;
+    // workspace of BVH builds, kept from one to the next (bvh_build.hip)
+    void* build_ws = nullptr;
+    size_t build_ws_bytes = 0;
     // persistent-kernel work counters
     uint32_t* counters = nullptr;  // 64 words
     // scratch for raw trace calls with host pointers
