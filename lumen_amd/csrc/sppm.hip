@@ -313,12 +313,12 @@ __global__ __launch_bounds__(256) void k_sppm_bounds(const float* __restrict__ s
 // A light path between two bounces (sppm_light.rgen:43-114), of pixel slot q
 // (x = q % W, y = q / W).
 struct LightState {
-    f3 pos, wi, thr;
+    f3 thr;
     uint32_t q, rng;
     int depth;
 };
 
-LT_DEV void light_begin(const SceneView& sv, const SppmLaunch& L, uint32_t q, LightState& s) {
+LT_DEV void light_begin(const SceneView& sv, const SppmLaunch& L, uint32_t q, LightState& s, PathRay& r) {
     RNG seed = {q % L.width, q / L.width, L.word, 0u};
     f4 rp;
     rp.x = rnd(seed);
@@ -329,26 +329,24 @@ LT_DEV void light_begin(const SceneView& sv, const SppmLaunch& L, uint32_t q, Li
     float cos_theta, pdf_pos, pdf_dir;
     uint32_t flags, li;
     f3 n;
-    const f3 Le = sample_light_Le(sv, rp, rd0, rd1, cos_theta, flags, li, s.pos, s.wi, n, pdf_pos, pdf_dir);
-    const float abs_cos = fabsf(dot(n, s.wi));
+    const f3 Le = sample_light_Le(sv, rp, rd0, rd1, cos_theta, flags, li, r.o, r.d, n, pdf_pos, pdf_dir);
+    const float abs_cos = fabsf(dot(n, r.d));
     s.thr = (abs_cos == 0.0f || pdf_dir <= 0.0f) ? mk3(0.0f) : Le * abs_cos / (pdf_dir * pdf_pos);
     s.q = q;
     s.rng = seed.w;
     s.depth = 0;
 }
 
-// One bounce; false once the path has ended.
-template <bool COUNT>
+// One bounce, from the closest hit h of the ray along wi to the next ray; false
+// once the path has ended.
 LT_DEV bool light_step(const SceneView& sv, const SppmLaunch& L, const SppmGrid& g, LightState& s,
                        SppmPhoton* __restrict__ photons, uint32_t* __restrict__ key, uint32_t* __restrict__ count,
-                       const TraceStack& stk, Ctr& c) {
+                       const HitRec& h, f3 wi, PathRay& r) {
     const int depth = s.depth++;
+    if (h.gid == 0xFFFFFFFFu) return false;
     Payload pl;
-    if (COUNT) c.closest++;
-    HitRec h;
-    if (!trace_bvh<false, COUNT>(sv, s.pos, s.wi, SPPM_TMIN, SPPM_TMAX, h, stk, c.nodes, c.tris)) return false;
     fill_payload(sv, h.inst, h.prim, h.u, h.v, pl);
-    const f3 wo = -s.wi;
+    const f3 wo = -wi;
     f3 n_s = pl.n_s, n_g = pl.n_g;
     bool side = true;
     if (dot(pl.n_g, wo) < 0.0f) n_g = -n_g;
@@ -364,16 +362,16 @@ LT_DEV bool light_step(const SceneView& sv, const SppmLaunch& L, const SppmGrid&
         const uint32_t ref = s.q * (uint32_t)L.max_depth + (uint32_t)depth;
         SppmPhoton& ph = photons[ref];
         ph.a = make_float4(pl.pos.x, pl.pos.y, pl.pos.z, __uint_as_float((uint32_t)depth + 1u));
-        ph.b = make_float4(-s.wi.x, -s.wi.y, -s.wi.z, s.thr.x);
+        ph.b = make_float4(-wi.x, -wi.y, -wi.z, s.thr.x);
         ph.c = make_float4(s.thr.y, s.thr.z, 0.0f, 0.0f);
         atomicMax(&key[hb], ref + 1u);
         atomicAdd(&count[hb], 1u);
     }
-    s.pos = offset_ray(pl.pos, n_g);
+    r.o = offset_ray(pl.pos, n_g);
     float pdf, cos_t;
     RNG seed = {s.q % L.width, s.q / L.width, L.word, s.rng};
     const float r0 = rnd(seed), r1 = rnd(seed), r2 = rnd(seed);
-    const f3 f = sample_bsdf(n_s, wo, mat, 0u, side, s.wi, pdf, cos_t, r0, r1, r2);
+    const f3 f = sample_bsdf(n_s, wo, mat, 0u, side, r.d, pdf, cos_t, r0, r1, r2);
     s.thr *= f * fabsf(cos_t) / pdf;
     if ((f.x == 0.0f && f.y == 0.0f && f.z == 0.0f) || pdf == 0.0f) return false;
     if (depth > RR_MIN_DEPTH) {
@@ -388,8 +386,7 @@ LT_DEV bool light_step(const SceneView& sv, const SppmLaunch& L, const SppmGrid&
 #ifndef LT_SPPM_LIGHT_WAVES
 #define LT_SPPM_LIGHT_WAVES 4
 #endif
-// persistent lanes: one bounce per iteration, a lane takes the next path as
-// soon as its own ends
+// a lane takes the next path as soon as its own ends (stream_paths)
 template <bool COUNT>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_SPPM_LIGHT_WAVES))) void k_sppm_light(
     SceneView sv, SppmLaunch L, const SppmBounds* __restrict__ bounds, SppmPhoton* __restrict__ photons,
@@ -401,21 +398,20 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     const SppmGrid g = sppm_grid(*bounds);
     Ctr c{0, 0, 0, 0};
     LightState s;
-    bool has = false;
-    WaveTiles wt = wave_tiles(L.n_px, work);
-    for (;;) {
-        const unsigned long long idle = __ballot(!has);
-        const uint32_t n_idle = (uint32_t)__popcll(idle);
-        if (n_idle == 64u || (!wt.done && n_idle >= L.regen_min)) {
-            if (n_idle == 64u && wt.done) break;
-            uint32_t q = 0u;
-            if (take_items(wt, idle, q)) {
-                light_begin(sv, L, q, s);
-                has = true;
-            }
-        }
-        if (has && !light_step<COUNT>(sv, L, g, s, photons, key, count, stk, c)) has = false;
-    }
+    auto ray = [&](PathRay& r) {
+        r.tmin = SPPM_TMIN;
+        r.tmax = SPPM_TMAX;
+        if (COUNT) c.closest++;
+        return true;
+    };
+    auto begin = [&](uint32_t q, PathRay& r) {
+        light_begin(sv, L, q, s, r);
+        return ray(r);
+    };
+    auto shade = [&](const TraceState& t, PathRay& r) {
+        return light_step(sv, L, g, s, photons, key, count, t.best, t.d, r) && ray(r);
+    };
+    stream_paths<COUNT>(sv, stk, wave_tiles(L.n_px, work), shade, begin, c);
     if (COUNT) flush_counts(c, counts);
 }
 
