@@ -15,11 +15,9 @@ struct lt_adjoint {
     lt_adjoint_config cfg{};
     uint32_t aw = 0, ah = 0, rw = 0, rh = 0;
     uint32_t tiles_x = 0, n_items = 0;
-    uint32_t blocks = 0;
     // private to this object so that it may run on a caller's stream next
     // to the context's own work
-    uint32_t* work = nullptr;   // persistent-grid work counter
-    uint32_t* spill = nullptr;  // traversal stack spill of the resident threads
+    AdjWork w{};
     // counting mode: kCountSlots counters of the last forward / backward call
     unsigned long long* counts = nullptr;
     bool counting = false;
@@ -83,6 +81,7 @@ void fill_launch(const lt_adjoint* a, const lt_camera* cam, uint32_t seed, AdjLa
     L.tiles_x = a->tiles_x;
     L.n_items = a->n_items;
     L.rec_depth = adj_rec_depth(a->cfg.max_depth);
+    L.trunk_depth = adj_trunk_depth(a->cfg.max_depth, a->cfg.variants);
 }
 
 // the scene may have been replaced since create: the texture grids the
@@ -128,11 +127,25 @@ lt_status lt_adjoint_create(lt_context* ctx, const lt_adjoint_config* cfg, lt_ad
     a->rh = rh;
     a->tiles_x = (uint32_t)tiles_x;
     a->n_items = (uint32_t)items;
-    a->blocks = (uint32_t)ctx->num_cus * std::max(1u, ctx->tuning.path_blocks_per_cu);
     (void)hipSetDevice(ctx->device);
-    hipError_t e = hipMalloc(&a->work, 256);
+    a->w.blocks = adjoint_blocks(ctx);
+    hipError_t e = hipMalloc(&a->w.work, 256);
     if (e == hipSuccess)
-        e = hipMalloc(&a->spill, (size_t)a->blocks * kTraceBlock * (ltb::kStackTotal - ltb::kLdsStack) * sizeof(uint32_t));
+        e = hipMalloc(&a->w.spill, (size_t)a->w.blocks * kTraceBlock * (ltb::kStackTotal - ltb::kLdsStack) * sizeof(uint32_t));
+    // without these two the kernels do the same work unshared
+    const size_t trunk = adj_trunk_words4(adj_trunk_depth(c.max_depth, c.variants));
+    const size_t texels = adj_texel_floats((uint64_t)c.width * c.height, c.spp, c.variants,
+                                           c.albedo_texture >= 0 ? (uint64_t)aw * ah : 0u,
+                                           c.roughness_texture >= 0 ? (uint64_t)rw * rh : 0u);
+    if (e == hipSuccess && trunk &&
+        hipMalloc(&a->w.trunk, (size_t)a->w.blocks * (kTraceBlock / 64) * trunk * sizeof(uint4)) != hipSuccess) {
+        (void)hipGetLastError();
+        a->w.trunk = nullptr;
+    }
+    if (e == hipSuccess && texels && hipMalloc(&a->w.texels, texels * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        a->w.texels = nullptr;
+    }
     if (e != hipSuccess) {
         lt_adjoint_destroy(a);
         return lt_hip_check(ctx, e, "lt_adjoint_create: hipMalloc");
@@ -145,8 +158,10 @@ lt_status lt_adjoint_destroy(lt_adjoint* a) {
     if (!a) return LT_ERR_INVALID_ARG;
     (void)hipSetDevice(a->ctx->device);
     (void)hipDeviceSynchronize();
-    if (a->work) (void)hipFree(a->work);
-    if (a->spill) (void)hipFree(a->spill);
+    if (a->w.work) (void)hipFree(a->w.work);
+    if (a->w.spill) (void)hipFree(a->w.spill);
+    if (a->w.trunk) (void)hipFree(a->w.trunk);
+    if (a->w.texels) (void)hipFree(a->w.texels);
     if (a->counts) (void)hipFree(a->counts);
     delete a;
     return LT_OK;
@@ -179,7 +194,7 @@ lt_status lt_adjoint_forward(lt_adjoint* a, const lt_camera* cam, uint32_t seed,
     AdjLaunch L{};
     fill_launch(a, cam, seed, L);
     AdjBuffers B{albedo, roughness, images, sample_cache, nullptr, nullptr, nullptr};
-    return launch_adjoint(ctx, L, B, false, a->work, a->spill, a->blocks, a->counting ? a->counts : nullptr,
+    return launch_adjoint(ctx, L, B, false, a->w, a->counting ? a->counts : nullptr,
                           (hipStream_t)stream);
 }
 
@@ -197,7 +212,7 @@ lt_status lt_adjoint_backward(lt_adjoint* a, const lt_camera* cam, uint32_t seed
     AdjLaunch L{};
     fill_launch(a, cam, seed, L);
     AdjBuffers B{albedo, roughness, nullptr, (float*)sample_cache, d_images, grad_albedo, grad_roughness};
-    return launch_adjoint(ctx, L, B, true, a->work, a->spill, a->blocks, a->counting ? a->counts : nullptr,
+    return launch_adjoint(ctx, L, B, true, a->w, a->counting ? a->counts : nullptr,
                           (hipStream_t)stream);
 }
 

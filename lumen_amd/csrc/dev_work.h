@@ -17,14 +17,19 @@
 
 namespace ltd {
 
-// per cent of the tiles dealt out beforehand (at least one round)
-#ifndef LT_STATIC_PCT
-#define LT_STATIC_PCT 60
-#endif
+// Per cent of the tiles dealt out beforehand (at least one round).  Ray
+// batches, BDPT, VCM and SPPM lose 1-4 % with 45 (2.07M bounce rays 624 ->
+// 633 us, SPPM 13.9 -> 14.5 ms) and more with 25.  Images of paths and of
+// texture variants (`image` below) have dear and cheap regions that a wave's
+// dealt tiles may keep hitting: 60 -> 45 takes 16 Path frames of 509x383 from
+// 1.79 to 1.62 ms and the adjoint at 512x512 from 53.0 to 49.0 ms (90 %: 72
+// ms), and a 1080p Path frame is even.
+constexpr uint32_t kStaticPct = 60;
+constexpr uint32_t kStaticPctImage = 45;
 
 // Rounds of one tile per wave that need no counter.
-__host__ __device__ inline uint32_t static_rounds(uint32_t n_tiles, uint32_t n_waves) {
-    const uint32_t r = (uint32_t)((uint64_t)n_tiles * LT_STATIC_PCT / 100u / n_waves);
+__host__ __device__ inline uint32_t static_rounds(uint32_t n_tiles, uint32_t n_waves, bool image) {
+    const uint32_t r = (uint32_t)((uint64_t)n_tiles * (image ? kStaticPctImage : kStaticPct) / 100u / n_waves);
     return r ? r : 1u;
 }
 
@@ -37,9 +42,9 @@ inline uint32_t work_blocks(uint64_t n_items, uint32_t blocks, uint32_t waves_pe
     return (uint32_t)(up < blocks ? up : blocks);
 }
 // true if that grid takes tiles from the counter, which must then start at zero
-inline bool work_counted(uint64_t n_items, uint32_t blocks, uint32_t waves_per_block) {
+inline bool work_counted(uint64_t n_items, uint32_t blocks, uint32_t waves_per_block, bool image = false) {
     const uint32_t tiles = (uint32_t)((n_items + 63u) / 64u), waves = blocks * waves_per_block;
-    return static_rounds(tiles, waves) * (uint64_t)waves < tiles;
+    return static_rounds(tiles, waves, image) * (uint64_t)waves < tiles;
 }
 
 // The wave's part of the items; every field is wave-uniform.
@@ -55,16 +60,23 @@ struct WaveTiles {
 
 // Call with the whole wave active.  Workgroups are dealt to the 8 XCDs round
 // robin (blockIdx mod 8), each with its own L2: the waves of one XCD are
-// numbered consecutively, so that a round gives it one run of tiles.
-LT_DEV WaveTiles wave_tiles(uint32_t n_items, uint32_t* work) {
+// numbered consecutively, so that a round gives it one run of tiles.  Where
+// regions of an image differ in cost that would give one XCD, or one CU, all
+// the dear ones: with `image` neighbouring tiles go to different workgroups
+// instead (a 160x120 preview frame 252 -> 237 us; the adjoint at 256x200, 3
+// variants: 5.12 -> 3.93 ms; a 1080p Path frame even).
+LT_DEV WaveTiles wave_tiles(uint32_t n_items, uint32_t* work, bool image = false) {
     WaveTiles t;
     const uint32_t wpb = blockDim.x >> 6, wib = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     t.stride = gridDim.x * wpb;
-    t.next = (gridDim.x & 7u) == 0u ? ((blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3)) * wpb + wib
+    if (image)
+        t.next = wib * gridDim.x + blockIdx.x;
+    else
+        t.next = (gridDim.x & 7u) == 0u ? ((blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3)) * wpb + wib
                                     : blockIdx.x * wpb + wib;
     t.n_items = n_items;
     t.n_tiles = (n_items + 63u) >> 6;
-    t.n_static = static_rounds(t.n_tiles, t.stride) * t.stride;
+    t.n_static = static_rounds(t.n_tiles, t.stride, image) * t.stride;
     t.base = t.left = 0u;
     t.done = false;
     t.work = work;

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     Ctr c{0, 0, 0, 0};
     PathState p;
     bool has = false;
-    WaveTiles wt = wave_tiles(n_items, work);
+    WaveTiles wt = wave_tiles(n_items, work, true);
     for (;;) {
         const unsigned long long idle = __ballot(!has);
         const uint32_t n_idle = (uint32_t)__popcll(idle);
@@ -238,7 +238,7 @@ lt_status launch_path_persistent(lt_context* ctx, PathSamples& ps, const PathLau
         L.spp = std::min(group, L0.spp - f);
         L.regen_min = ctx->tuning.regen_min ? ctx->tuning.regen_min : 4u;
         const uint32_t grid = work_blocks(items * L.spp, (uint32_t)blocks, kTraceBlock / 64);
-        if (work_counted(items * L.spp, grid, kTraceBlock / 64))
+        if (work_counted(items * L.spp, grid, kTraceBlock / 64, true))
             hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 1u);
         if (count)
             hipLaunchKernelGGL((k_path_regen<true>), dim3(grid), dim3(kTraceBlock), 0, ctx->stream, sv, L, accum,
