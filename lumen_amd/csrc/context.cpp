@@ -70,10 +70,10 @@ lt_status ensure_spill(lt_context* ctx, size_t threads) {
 }
 
 uint32_t resident_blocks(const void* kernel, uint32_t fixed) {
-    if (fixed) return fixed;
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kTraceBlock, 0) != hipSuccess || n < 1) return 1u;
-    return (uint32_t)n;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kTraceBlock, 0) != hipSuccess || n < 1)
+        return fixed ? fixed : 1u;
+    return fixed ? std::min(fixed, (uint32_t)n) : (uint32_t)n;
 }
 
 static void free_scene(DeviceScene& s) {

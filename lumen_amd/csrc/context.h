@@ -150,7 +150,8 @@ constexpr int kMaxPhases = 8;
 // timing is on (at most kMaxPhases phases)
 void phase_mark(lt_context* ctx);
 // workgroups of kTraceBlock threads of `kernel` that one CU holds at once
-// (its register and LDS use), at least 1; `fixed` (a tuning value) wins if set
+// (its register and LDS use), at least 1; `fixed` (a tuning value, if set) can
+// only lower it: work is dealt out to waves that all have to run at once
 uint32_t resident_blocks(const void* kernel, uint32_t fixed);
 
 // builder / kernels (implemented in the .hip files)

@@ -12,11 +12,13 @@
 //     shade[d]    emission, light sample (shadow record), MIS-BSDF record for
 //                 area lights, BSDF sample + Russian roulette -> extend queue d+1
 //   accumulate    running mean into the output (path.rgen:102-112)
-// Terminated paths leave the queues (ballot + one atomic per wave), so every
+// Terminated paths leave the queues (one atomic per workgroup), so every
 // stage runs on full waves whatever the path lengths.  Each path consumes its
 // pcg4d stream in exactly the order of path.rgen / pt_commons.glsl, so the
 // image equals the persistent kernel's up to float summation order.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "context.h"
 #include "dev_atmosphere.h"
@@ -36,32 +38,39 @@ constexpr int RR_MIN_DEPTH = 3;        // path.rgen:21
 // frame number of frame f of the launch
 LT_DEV uint32_t frame_of(const PathLaunch& L, uint32_t f) { return (L.frame_dev ? *L.frame_dev : L.frame_start) + f; }
 
-// wave-level compaction: returns this lane's slot in `queue` (one atomic per wave)
-LT_DEV uint32_t wave_append(uint32_t* len, bool pred) {
-    const unsigned long long mask = __ballot(pred);
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t n = __popcll(mask);
-    uint32_t base = 0;
-    const int leader = __ffsll((long long)mask) - 1;
-    if (n && (int)lane == leader) base = atomicAdd(len, n);
-    base = __shfl(base, leader < 0 ? 0 : leader);
-    const unsigned long long below = mask & ((1ull << lane) - 1ull);
-    return base + (uint32_t)__popcll(below);
+// Workgroup-level compaction into the three queues a shade stage fills: this
+// thread's slot in each.  One atomic per queue and 256 items, as every atomic
+// on a counter takes its turn of about 10 ns (per wave: 0.15 ms a stage of a
+// 1200x800 frame).  Two buffers of s, used in turn, let a wave begin the next
+// append while another still reads this one.  The whole workgroup must call.
+constexpr uint32_t kShadeBlock = 256, kShadeWaves = kShadeBlock / 64;
+struct AppendLds {
+    uint32_t n[2][3][kShadeWaves];
+    uint32_t base[2][3];
+};
+LT_DEV void block_append(AppendLds& s, uint32_t buf, uint32_t* const (&len)[3], const bool (&want)[3],
+                         uint32_t (&slot)[3]) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const unsigned long long mask = __ballot(want[k]);
+        slot[k] = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+        if (lane == 0u) s.n[buf][k][wave] = (uint32_t)__popcll(mask);
+    }
+    __syncthreads();
+    if (threadIdx.x < 3u) {
+        uint32_t total = 0u;
+        for (uint32_t w = 0; w < kShadeWaves; w++) total += s.n[buf][threadIdx.x][w];
+        uint32_t* const l = threadIdx.x == 0u ? len[0] : threadIdx.x == 1u ? len[1] : len[2];
+        s.base[buf][threadIdx.x] = total ? atomicAdd(l, total) : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        slot[k] += s.base[buf][k];
+        for (uint32_t w = 0; w < wave; w++) slot[k] += s.n[buf][k][w];
+    }
 }
-
-// Persistent wave loop helper: a wave takes 64 consecutive items.
-#define WAVE_LOOP(n_expr, work_ptr)                         \
-    const uint32_t lane = threadIdx.x & 63u;                \
-    const uint32_t n_items = (n_expr);                      \
-    for (;;) {                                              \
-        uint32_t base = 0;                                  \
-        if (lane == 0) base = atomicAdd((work_ptr), 64u);   \
-        base = __shfl(base, 0);                             \
-        if (base >= n_items) break;                         \
-        const uint32_t item = base + lane;                  \
-        const bool active = item < n_items;
-
-#define WAVE_LOOP_END }
 
 __global__ void k_wf_reset(WaveCtl* ctl) {
     uint32_t* p = (uint32_t*)ctl;
@@ -99,14 +108,21 @@ __global__ __launch_bounds__(256) void k_wf_generate(PathLaunch L, uint32_t f, W
 #define LT_WF_SHADE_WAVES 1
 #endif
 template <bool COUNT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LT_WF_SHADE_WAVES))) void k_wf_shade(SceneView sv, PathLaunch L, uint32_t f, WaveState S,
+__global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(LT_WF_SHADE_WAVES))) void k_wf_shade(SceneView sv, PathLaunch L, uint32_t f, WaveState S,
                                                   WaveCtl* ctl, uint32_t depth, uint32_t sorted,
                                                   unsigned long long* __restrict__ counts) {
     const uint32_t frame_word = frame_of(L, f) ^ L.seed;
     const uint32_t* q = sorted ? S.sorted : S.queue[depth & 1];
     uint32_t* qn = S.queue[(depth + 1) & 1];
     uint32_t n_closest = 0, n_shadow = 0;
-    WAVE_LOOP(ctl->q_len[depth], &ctl->work[depth][1])
+    __shared__ AppendLds s_append;
+    // items dealt round robin, no counter: one atomic per wave of the full grid
+    // alone was 0.09 ms a stage
+    const uint32_t n_items = ctl->q_len[depth];
+    uint32_t buf = 0u;
+    for (uint32_t first = blockIdx.x * kShadeBlock; first < n_items; first += gridDim.x * kShadeBlock) {
+    const uint32_t item = first + threadIdx.x;
+    const bool active = item < n_items;
     bool cont = false, want_sh = false, want_mis = false;
     uint32_t p = 0;
     ShadowRec sr;
@@ -224,20 +240,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LT_WF_SHADE
         counter = seed.w;
         S.col[p] = make_float4(c.x, c.y, c.z, 0.0f);
     }
-    // queue appends (every lane of the wave takes part in the ballots)
-    const uint32_t ssh = wave_append(&ctl->sh_len[depth], want_sh);
-    if (want_sh) S.shadow[ssh] = sr;
-    const uint32_t smis = wave_append(&ctl->mis_len[depth], want_mis);
-    if (want_mis) S.mis[smis] = mr;
-    const uint32_t sn = wave_append(&ctl->q_len[depth + 1], cont);
+    uint32_t* const len[3] = {&ctl->sh_len[depth], &ctl->mis_len[depth], &ctl->q_len[depth + 1]};
+    const bool want[3] = {want_sh, want_mis, cont};
+    uint32_t slot[3];
+    block_append(s_append, buf, len, want, slot);
+    buf ^= 1u;
+    if (want_sh) S.shadow[slot[0]] = sr;
+    if (want_mis) S.mis[slot[1]] = mr;
     if (cont) {
-        qn[sn] = p;
+        qn[slot[2]] = p;
         S.ray_o[p] = new_o;
         S.ray_d[p] = new_d;
         S.thr[p] = thr4;
     }
     if (active) S.meta[p] = make_uint4(counter, last_spec, 0u, 0u);
-    WAVE_LOOP_END
+    }
     if (COUNT) {
         unsigned long long a = n_closest, b = n_shadow;
         for (int o = 32; o > 0; o >>= 1) {
@@ -501,10 +518,13 @@ lt_status launch_path_wavefront(lt_context* ctx, WaveBuffers& wb, const PathLaun
     if (L.max_depth > kWaveMaxDepth) return lt_fail(ctx, LT_ERR_UNSUPPORTED, "wavefront max_depth above 32");
     lt_status st = wave_alloc(ctx, wb, n);
     if (st != LT_OK) return st;
-    const size_t tblocks = (size_t)ctx->num_cus * ctx->tuning.path_blocks_per_cu;
+    // no more waves than run at once, as their rays are dealt out beforehand
+    const uint32_t resident = std::max(1u, std::min(ctx->tuning.path_blocks_per_cu,
+                                                    resident_blocks(reinterpret_cast<const void*>(&k_wf_trace<false>), 0u)));
+    const size_t tblocks = work_blocks((uint64_t)n * 3u, (uint32_t)ctx->num_cus * resident, kTraceBlock / 64);
     st = ensure_spill(ctx, tblocks * kTraceBlock);
     if (st != LT_OK) return st;
-    const size_t sblocks = (size_t)ctx->num_cus * 8;
+    const size_t sblocks = std::min<size_t>((size_t)ctx->num_cus * 8, (n + kShadeBlock - 1) / kShadeBlock);
     const uint32_t sort = ctx->tuning.wf_sort == LT_WF_SORT_BSDF ? 1u : 0u;
     SceneView sv = make_scene_view(ctx);
     auto* cnt = (unsigned long long*)d_counts;
@@ -530,10 +550,10 @@ lt_status launch_path_wavefront(lt_context* ctx, WaveBuffers& wb, const PathLaun
                 hipLaunchKernelGGL(k_wf_bin_scatter, dim3(sblocks), dim3(256), 0, ctx->stream, wb.S, wb.ctl, d);
             }
             if (count)
-                hipLaunchKernelGGL((k_wf_shade<true>), dim3(sblocks), dim3(256), 0, ctx->stream, sv, L, f, wb.S,
+                hipLaunchKernelGGL((k_wf_shade<true>), dim3(sblocks), dim3(kShadeBlock), 0, ctx->stream, sv, L, f, wb.S,
                                    wb.ctl, d, sort, cnt);
             else
-                hipLaunchKernelGGL((k_wf_shade<false>), dim3(sblocks), dim3(256), 0, ctx->stream, sv, L, f, wb.S,
+                hipLaunchKernelGGL((k_wf_shade<false>), dim3(sblocks), dim3(kShadeBlock), 0, ctx->stream, sv, L, f, wb.S,
                                    wb.ctl, d, sort, cnt);
         }
         hipLaunchKernelGGL(k_wf_accumulate, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, L, f, wb.S, accum);

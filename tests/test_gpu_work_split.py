@@ -57,3 +57,25 @@ def test_frames_of_one_launch_equal_single_frames(gpu_ctx, strategy, size):
         it.destroy()
     assert np.array_equal(imgs[0], imgs[1]) and np.array_equal(imgs[0], imgs[2])
     assert np.isfinite(imgs[0]).all() and (imgs[0][..., 3] == 1).all()
+
+
+@pytest.mark.parametrize("size", [(1, 1), (17, 15), (16, 16), (257, 1), (509, 383)])
+def test_wavefront_queues_around_a_workgroup(gpu_ctx, size):
+    """Queues of one item to many workgroups' worth: the wavefront form equals
+    the persistent one up to float summation order (test_gpu_path.py's bound),
+    and repeats itself bit for bit (a path's terms do not depend on its
+    queue slot)."""
+    print(f"[gpu] wavefront queues {size}", flush=True)
+    sc = la.Scene.procedural("cornell", seed=1)
+    imgs = []
+    for strategy in ("wavefront", "wavefront", "persistent"):
+        it = la.Path(sc, gpu_ctx, size[0], size[1], strategy=strategy)
+        it.seed = 5
+        it.init()
+        it.create_accel()
+        it.render(spp=3)
+        it.update()
+        imgs.append(it.output_tex)
+        it.destroy()
+    assert np.array_equal(imgs[0], imgs[1])
+    np.testing.assert_allclose(imgs[0], imgs[2], rtol=1e-4, atol=1e-5)
