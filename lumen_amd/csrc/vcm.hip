@@ -531,8 +531,10 @@ LT_DEV uint32_t cell_pack(int x, int y, int z) {
 // waits on another lane's serial loop.  The wave's sum is added to the
 // pixel's colour with float atomics (the order of the sum is the only
 // difference from a serial loop).
+// Four waves per SIMD: the loads of photons wait on HBM and L2 (8 frames of the
+// caustics scene, 1024x1024: 30.9 ms with three, 30.2 with four).
 #ifndef LT_VCM_MERGE_WAVES
-#define LT_VCM_MERGE_WAVES 3
+#define LT_VCM_MERGE_WAVES 4
 #endif
 #ifndef LT_VCM_CELL_DIV
 #define LT_VCM_CELL_DIV 2
