@@ -313,8 +313,7 @@ typedef struct lt_tuning {
                                       depth grouped by the BSDF type of their material
                                       before shading); 0 = unchanged                     */
     uint32_t xcd_bands;            /* LT_XCD_BANDS_OFF (default) or LT_XCD_BANDS_ON; kept
-                                      and returned, no effect: the tiles of a round are
-                                      always dealt in one run per XCD; 0 = unchanged     */
+                                      and returned, no effect; 0 = unchanged             */
     uint32_t reserved[8];
 } lt_tuning;
 #define LT_WF_SORT_NONE 1u
