@@ -464,7 +464,7 @@ typedef struct lt_render_stats {
     uint64_t shadow_tris_tested;
     /* With lt_render_set_timing on: device time of each phase of the first
      * frame of the last lt_render.  Phases: Path persistent / megakernel: 1
-     * (the frame); Path wavefront: 1; BDPT: walk and connect of each pixel
+     * (the frame); Path wavefront: 1; BDPT: walk (with the MIS prefixes) and connect of each pixel
      * chunk (one chunk at 1024x1024, depth 8), then the splat resolve; VCM: 4 (light pass + photon grid, eye pass, merge pass,
      * resolve; the last two 0 without the corrected estimator's merging);
      * SPPM: 4 (eye pass, grid bounds, light pass, gather). */
@@ -561,7 +561,9 @@ lt_status lt_adjoint_backward(lt_adjoint* adj, const lt_camera* camera, uint32_t
  * forward and backward calls run the counting variants of their kernels and
  * record the work of the call; lt_adjoint_counts waits for the device and
  * returns that of the last call: closest-hit rays, occlusion rays, BVH8 nodes
- * and triangles visited by all queries, and those of the occlusion queries. */
+ * and triangles visited by all queries, and those of the occlusion queries.
+ * A ray that several variants share counts once for each of them, the nodes
+ * and triangles it visits once. */
 lt_status lt_adjoint_set_counting(lt_adjoint* adj, int32_t on);
 lt_status lt_adjoint_counts(lt_adjoint* adj, uint64_t counts[6]);
 

@@ -221,12 +221,17 @@ lt_status launch_path_persistent(lt_context* ctx, PathSamples& ps, const PathLau
     const size_t n = (size_t)L0.width * L0.height;
     // frames per launch: what the sample buffer holds, and items that fit 32 bits
     const size_t items = (size_t)((L0.width + 7) / 8) * ((L0.height + 7) / 8) * 64;
-    const uint32_t group = (uint32_t)std::max<size_t>(
+    uint32_t group = (uint32_t)std::max<size_t>(
         1, std::min<size_t>({L0.spp, kPathSampleBytes / (n * sizeof(float4)), (1ull << 31) / items}));
     if (group > 1 && ps.capacity < group * n) {
         path_samples_free(ps);
-        LT_HIP(ctx, hipMalloc(&ps.rad, group * n * sizeof(float4)));
-        ps.capacity = group * n;
+        if (hipMalloc(&ps.rad, group * n * sizeof(float4)) == hipSuccess) {
+            ps.capacity = group * n;
+        } else {  // no room: frame by frame, which needs no buffer
+            (void)hipGetLastError();
+            ps.rad = nullptr;
+            group = 1;
+        }
     }
     SceneView sv = make_scene_view(ctx);
     auto* cnt = (unsigned long long*)d_counts;
