@@ -220,7 +220,11 @@ LT_DEV void trace_init(const SceneView& sv, TraceState& s, f3 o, f3 d, float tmi
     s.sp = 0;
     s.qn = 0;
     s.tri_base = s.tris = 0u;
-    s.next = sv.num_nodes != 0 ? 0u : kNoNode;
+    // a NaN in the origin or the direction, or an empty (or NaN) interval: no
+    // triangle can be hit, so no node is visited.  The node step could not tell:
+    // to its sign test a NaN distance is a hit, of every child of every node
+    const float e = s.rp.err.x + s.rp.err.y + s.rp.err.z;
+    s.next = sv.num_nodes != 0 && e == e && s.lo <= s.hi ? 0u : kNoNode;
 }
 
 // Processes one BVH8 node (its children's boxes; the hit leaves' triangles are
@@ -282,7 +286,7 @@ LT_DEV bool trace_step_dyn(const SceneView& sv, TraceState& s, const TraceStack&
             t0 = fmaxf(t0, s.lo);
             t1 = fminf(t1, s.hi);
             // (miss << 1) | sign(t1 - t0); equal distances give +0, a NaN (both
-            // infinite) the default positive one: a hit
+            // infinite; trace_init keeps others out) the default positive one: a hit
             miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(t1 - t0), 31);
         }
         const uint32_t hit_int = imask & ~miss;

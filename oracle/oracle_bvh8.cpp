@@ -75,7 +75,9 @@ extern "C" void ora_bvh8_trace(const void* nodes_v, uint32_t n_nodes, const void
             }
         }
         std::vector<uint32_t> stack;
-        if (n_nodes) stack.push_back(0);
+        // a ray with a NaN, or an empty interval, hits nothing and visits no node
+        const float Es = E[0] + E[1] + E[2];
+        if (n_nodes && Es == Es && tmin - margin <= tmax + margin) stack.push_back(0);
         while (!stack.empty() && !done) {
             const Node8h& nd = nodes[stack.back()];
             stack.pop_back();
