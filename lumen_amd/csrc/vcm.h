@@ -1,6 +1,7 @@
 // vcm.h — launch parameters and buffers of the VCM integrator kernels.
 #pragma once
 #include "context.h"
+#include "vcm_grid.h"
 
 constexpr int kVcmMaxDepth = 16;
 
@@ -19,7 +20,7 @@ struct VcmLaunch {
     float radius, eta_vcm, eta_vc, eta_vm;
     int32_t grid_res[3];
     float bmin[3], bmax[3];
-    float inv_ext[3];  // 1 / (bmax - bmin): the corrected estimator's grid (see k_vcm_scatter)
+    float inv_ext[3];  // the corrected estimator's grid (vcm_inv_ext)
     float sky_col[3];
     uint32_t use_vm;
     uint32_t corrected;  // 0: the reference estimator, 1: corrected VCM

@@ -93,9 +93,9 @@ LT_DEV void grid_idx(const VcmLaunch& L, f3 p, int o[3]) {
 // whose cell index is monotone in the position finds each of them exactly
 // once, so the cheaper multiply changes nothing but bucket membership.
 LT_DEV void grid_idx_fast(const VcmLaunch& L, f3 p, int o[3]) {
-    o[0] = (int)((p.x - L.bmin[0]) * L.inv_ext[0] * (float)L.grid_res[0]);
-    o[1] = (int)((p.y - L.bmin[1]) * L.inv_ext[1] * (float)L.grid_res[1]);
-    o[2] = (int)((p.z - L.bmin[2]) * L.inv_ext[2] * (float)L.grid_res[2]);
+    o[0] = vcm_cell(p.x, L.bmin[0], L.inv_ext[0], L.grid_res[0]);
+    o[1] = vcm_cell(p.y, L.bmin[1], L.inv_ext[1], L.grid_res[1]);
+    o[2] = vcm_cell(p.z, L.bmin[2], L.inv_ext[2], L.grid_res[2]);
 }
 
 // The corrected estimator's buckets: 8 cells that follow one another along z
@@ -103,7 +103,6 @@ LT_DEV void grid_idx_fast(const VcmLaunch& L, f3 p, int o[3]) {
 // then is 25 columns of one or two contiguous bucket ranges each, so one
 // step of a wave reads all its ranges (64 lanes, two words each) where a bucket
 // per cell took two steps of 64 scattered ones.
-constexpr int kRunBits = 3;
 LT_DEV uint32_t run_base(int x, int y, int run, uint32_t n) {
     const uint32_t h = ((uint32_t)x * 73856093u) ^ ((uint32_t)y * 19349663u) ^ ((uint32_t)run * 83492791u);
     return (h % ((10u * n) >> kRunBits)) << kRunBits;
@@ -536,9 +535,6 @@ LT_DEV uint32_t cell_pack(int x, int y, int z) {
 #ifndef LT_VCM_MERGE_WAVES
 #define LT_VCM_MERGE_WAVES 4
 #endif
-#ifndef LT_VCM_CELL_DIV
-#define LT_VCM_CELL_DIV 2
-#endif
 #ifndef LT_VCM_MERGE_UNROLL
 #define LT_VCM_MERGE_UNROLL 4
 #endif
@@ -630,9 +626,8 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
         grid_idx_fast(L, qpos - mk3(L.radius), lo);
         grid_idx_fast(L, qpos + mk3(L.radius), hi);
         // columns of cells along z, each in runs
-        const int r0 = lo[2] >> kRunBits, nr = (hi[2] >> kRunBits) - r0 + 1;
-        const int ny = hi[1] - lo[1] + 1;
-        const int ncells = (hi[0] - lo[0] + 1) * ny * nr;
+        const VcmRuns runs = vcm_runs(lo, hi);
+        const int r0 = runs.r0, nr = runs.nr, ny = runs.ny, ncells = runs.n;
         if (COUNT && !second) n_bytes += sizeof(VcmQuery) + 8ull * (unsigned long long)ncells;
         f3 part = mk3(0.0f);
         uint32_t head = 0u, pend = 0u;  // wave-uniform: ring position and fill
@@ -1119,13 +1114,19 @@ lt_status launch_vcm(lt_context* ctx, VcmBuffers& b, const VcmLaunch& L0, const 
         L.frame_num = frame_num + f;
         vcm_frame_words(seed, L.frame_num, &L.light_word, &L.eye_word);
         vcm_radius_grid(L.bmin, L.bmax, cfg.radius_factor, cfg.alpha, L.frame_num, &L.radius, L.grid_res);
-        for (int k = 0; k < 3; k++) L.inv_ext[k] = 1.0f / (L.bmax[k] - L.bmin[k]);
         // The corrected estimator's cells are LT_VCM_CELL_DIV times finer per
         // axis than the reference's (about r / LT_VCM_CELL_DIV wide): a query's
         // box of +-r then covers (2 LT_VCM_CELL_DIV + 1)^3 smaller cells whose
         // photons lie closer to the radius.  Its sums do not depend on the grid.
-        if (L.use_vm && L.corrected)
-            for (int k = 0; k < 3; k++) L.grid_res[k] *= LT_VCM_CELL_DIV;
+        if (L.use_vm)
+            for (int k = 0; k < 3; k++) {
+                if (L.corrected) {
+                    L.grid_res[k] *= LT_VCM_CELL_DIV;
+                    L.inv_ext[k] = vcm_inv_ext(L0.bmin[k], L0.bmax[k], L.radius, L.grid_res[k]);
+                } else {
+                    L.bmax[k] = vcm_reference_bmax(L0.bmin[k], L0.bmax[k], L.radius, L.grid_res[k]);
+                }
+            }
         const float r2 = L.radius * L.radius;
         L.eta_vcm = PI * r2 * (float)N;
         L.eta_vc = 1.0f / L.eta_vcm;

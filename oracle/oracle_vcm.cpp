@@ -80,6 +80,7 @@ struct VcmCtx {
     float radius, eta_vcm, eta_vc, eta_vm, screen_size, cam_area;
     int grid_res[3];
     vec3 bmin, bmax;
+    vec3 ext;  // bmax - bmin; infinite where a query would visit more than 2^20 cells (every position in cell 0)
     int use_vc, use_vm;
     bool corrected;
     vec3 sky;
@@ -92,10 +93,17 @@ struct VcmCtx {
 // vcm_commons.glsl:19-23 (the clamp's result is discarded there, so indices
 // can fall outside the grid)
 static inline void grid_idx(const VcmCtx& c, vec3 p, int o[3]) {
-    const vec3 q = (p - c.bmin) / (c.bmax - c.bmin);
+    const vec3 q = (p - c.bmin) / c.ext;
     o[0] = (int)(q.x * (float)c.grid_res[0]);
     o[1] = (int)(q.y * (float)c.grid_res[1]);
     o[2] = (int)(q.z * (float)c.grid_res[2]);
+}
+
+static void set_ext(VcmCtx& c) {
+    c.ext = c.bmax - c.bmin;
+    float* const e[3] = {&c.ext.x, &c.ext.y, &c.ext.z};
+    for (int k = 0; k < 3; k++)
+        if (*e[k] >= 0.0f && !(2.0f * c.radius / *e[k] * (float)c.grid_res[k] <= 1048576.0f)) *e[k] = INFINITY;
 }
 
 static bool occluded(const VcmCtx& c, vec3 o, vec3 d, float tmax, Counters* cnt) {
@@ -618,6 +626,7 @@ double ora_render_vcm(const lt_scene_desc* s, void* accel, const lt_camera* cam,
         uint32_t lw, ew;
         ora_vcm_words(p->seed, frame_num, &lw, &ew);
         ora_vcm_radius_grid(s, p->radius_factor, p->alpha, frame_num, &c.radius, c.grid_res);
+        set_ext(c);
         const float r2 = c.radius * c.radius;
         c.eta_vcm = PI * r2 * c.screen_size;
         c.eta_vc = c.use_vc == 1 ? 1.0f / c.eta_vcm : 0.0f;
@@ -719,6 +728,7 @@ int ora_vcm_grid_selfcheck(const lt_scene_desc* s, void* accel, const lt_camera*
     uint32_t lw, ew;
     ora_vcm_words(p->seed, p->frame_start, &lw, &ew);
     ora_vcm_radius_grid(s, p->radius_factor, p->alpha, p->frame_start, &c.radius, c.grid_res);
+    set_ext(c);
     c.eta_vcm = PI * c.radius * c.radius * c.screen_size;
     c.eta_vc = 1.0f / c.eta_vcm;
     c.eta_vm = c.eta_vcm;
