@@ -28,6 +28,7 @@
 
 #include <algorithm>
 
+#include "alloc_set.h"
 #include "dev_scene.h"
 #include "dev_count.h"
 #include "dev_trace.h"
@@ -1094,10 +1095,17 @@ lt_status launch_vcm(lt_context* ctx, VcmBuffers& b, const VcmLaunch& L0, const 
     // corrected estimator with merging: a merge pass over the eye pass's queries
     const bool merge_pass = L0.use_vm && L0.corrected;
     if (merge_pass && !b.queries) {
-        LT_HIP(ctx, hipMalloc(&b.fcol, (size_t)b.n_paths * sizeof(float4)));
-        LT_HIP(ctx, hipMalloc(&b.queries, (size_t)kQuerySegs * query_seg_cap(L0) * sizeof(VcmQuery)));
-        LT_HIP(ctx, hipMalloc(&b.tasks, (size_t)kQuerySegs * kMergeTasks * sizeof(uint2)));
-        LT_HIP(ctx, hipMalloc(&b.qctr, 2 * kQuerySegs * kQueryCtrStride * sizeof(uint32_t)));
+        const BufferReq set[] = {
+            {(void**)&b.fcol, (size_t)b.n_paths * sizeof(float4)},
+            {(void**)&b.queries, (size_t)kQuerySegs * query_seg_cap(L0) * sizeof(VcmQuery)},
+            {(void**)&b.tasks, (size_t)kQuerySegs * kMergeTasks * sizeof(uint2)},
+            {(void**)&b.qctr, 2 * kQuerySegs * kQueryCtrStride * sizeof(uint32_t)},
+        };
+        const int e = alloc_set(set, [](void** p, size_t n) { return hipMalloc(p, n); }, [](void* p) { (void)hipFree(p); });
+        if (e != 0) {
+            (void)hipGetLastError();  // it is reported here, not by the next launch
+            return lt_hip_check(ctx, (hipError_t)e, "VCM merge buffers");
+        }
     }
     const uint32_t merge_blocks = ctx->num_cus * resident_blocks(reinterpret_cast<const void*>(&k_vcm_merge<false>), 0u);
     SceneView sv = make_scene_view(ctx);
