@@ -27,11 +27,20 @@ struct VcmLaunch {
     uint32_t regen_min;  // light pass: idle lanes that trigger taking new paths
 };
 
-// The merge queries lie in segments, one counter each, on cache lines of their
-// own; tile t of the image writes segment t mod kQuerySegs.
-constexpr uint32_t kQuerySegs = 64;
-constexpr uint32_t kQueryCtrStride = 32;  // words between counters
-constexpr uint32_t kMergeTasks = 16384;   // merge tasks a segment's list holds
+// The merge queries lie in segments, one per XCD, with a counter each on a
+// cache line of its own; tile t of the image writes segment t mod kQuerySegs.
+// One segment per XCD and no more: the waves of an XCD then work on one short
+// run of queries at a time, those of a few tiles, whose photons its 4 MiB L2
+// holds.  8 segments per XCD let each of them work on 8 places at once
+// (1024x1024, radius factor 1, merge pass: Cornell box 18.0 against 12.2 ms,
+// caustics 1.83 against 1.73 ms); two per XCD lie between (12.3 ms, 3.96
+// against 3.69 ms at 1024x800, radius factor 0.4).  The eye pass's 50,000
+// appends a frame, about 10 ns each on one counter, are hidden behind it with
+// 8 counters as with 64.
+constexpr uint32_t kQuerySegs = 8;
+static_assert(kQuerySegs == 8, "one segment per XCD: k_vcm_merge takes a workgroup's from its XCD");
+constexpr uint32_t kQueryCtrStride = 32;   // words between counters
+constexpr uint32_t kMergeTasks = 131072;   // merge tasks a segment's list holds
 __host__ __device__ inline size_t query_seg_cap(const VcmLaunch& L) {
     const size_t tiles = (size_t)((L.width + 7) / 8) * ((L.height + 7) / 8);
     return (tiles + kQuerySegs - 1) / kQuerySegs * 64 * (size_t)L.max_depth;

@@ -531,10 +531,12 @@ LT_DEV uint32_t cell_pack(int x, int y, int z) {
 // waits on another lane's serial loop.  The wave's sum is added to the
 // pixel's colour with float atomics (the order of the sum is the only
 // difference from a serial loop).
-// Four waves per SIMD: the loads of photons wait on HBM and L2 (8 frames of the
-// caustics scene, 1024x1024: 30.9 ms with three, 30.2 with four).
+// Three waves per SIMD (no scratch): four (128 VGPRs, 76 B of scratch per lane)
+// take 5 % off the caustics scene's pass, whose photons come from few places
+// (1024x1024: 1.73 -> 1.64 ms), and add 9 % on a closed diffuse scene (Cornell
+// box 12.2 -> 13.3 ms; 1024x800, radius factor 0.4: 3.70 -> 4.06 ms).
 #ifndef LT_VCM_MERGE_WAVES
-#define LT_VCM_MERGE_WAVES 4
+#define LT_VCM_MERGE_WAVES 3
 #endif
 #ifndef LT_VCM_MERGE_UNROLL
 #define LT_VCM_MERGE_UNROLL 4
@@ -576,28 +578,21 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     const uint64_t below = (1ull << lane) - 1ull;
     const float r2 = L.radius * L.radius;
     const float norm = 1.0f / (PI * r2 * (float)L.n_paths);
-    // The queries lie in kQuerySegs segments, tiles s, s + kQuerySegs, ... of
-    // the image in segment s.  Workgroups are dealt to the 8 XCDs round-robin
-    // (blockIdx mod 8), each XCD with its own L2: the waves of one XCD serve 8
-    // neighbouring segments, so at any time they work on a run of 8
-    // neighbouring tiles whose bucket ranges and photons its L2 then holds;
-    // within a segment they take every n-th query (neighbouring queries cost
-    // alike, so this balances).  Giving each XCD one contiguous eighth of all
-    // queries instead left the XCDs unevenly loaded (3.27 against 2.51 ms per
-    // caustics frame).
+    // Workgroups are dealt to the 8 XCDs round-robin (blockIdx mod 8), and the
+    // waves of XCD s serve segment s, the queries of tiles s, s + 8, ... of the
+    // image, taking every n-th query: at any time a run of neighbouring queries
+    // (they cost alike, so this balances), whose bucket ranges and photons the
+    // XCD's L2 then holds.  Giving each XCD one contiguous eighth of all queries
+    // instead left the XCDs unevenly loaded (3.27 against 2.51 ms per caustics
+    // frame).
     const uint32_t wpb = blockDim.x / 64u, wib = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64u));
     const uint32_t n_waves = gridDim.x * wpb;
-    uint32_t seg, q_first;
     const uint32_t q_stride = n_waves / kQuerySegs;
-    if ((gridDim.x & 7u) == 0u) {
-        const uint32_t w = (blockIdx.x >> 3) * wpb + wib;  // this wave within its XCD
-        seg = (blockIdx.x & 7u) * (kQuerySegs / 8u) + w % (kQuerySegs / 8u);
-        q_first = w / (kQuerySegs / 8u);
-    } else {
-        const uint32_t w = blockIdx.x * wpb + wib;
-        seg = w % kQuerySegs;
-        q_first = w / kQuerySegs;
-    }
+    // a grid that is no multiple of 8 only loses the match of segment and XCD
+    const bool by_xcd = (gridDim.x & 7u) == 0u;
+    const uint32_t w = blockIdx.x * wpb + wib;
+    const uint32_t seg = by_xcd ? blockIdx.x & 7u : w % kQuerySegs;
+    const uint32_t q_first = by_xcd ? (blockIdx.x >> 3) * wpb + wib : w / kQuerySegs;
     const uint32_t Q = q_first >= q_stride ? 0u
                        : second            ? min(n_tasks[seg * kQueryCtrStride], kMergeTasks)
                                            : n_queries[seg * kQueryCtrStride];
@@ -962,9 +957,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(LT_
     while (next_tile(wt)) {
         const uint32_t t = wt.base >> 6;
         const uint32_t x = (t % tiles_x) * 8 + (lane & 7), y = (t / tiles_x) * 8 + (lane >> 3);
-        // The queries of a tile go to the segment t mod kQuerySegs, which has a
-        // counter of its own: atomics on one counter are served one by one, 8-11
-        // ns each, and the eye pass appends about 50,000 times a frame.
+        // The queries of a tile go to the segment t mod kQuerySegs (vcm.h).
         const uint32_t seg = t % kQuerySegs;
         VcmQuery* tq = queries ? queries + (size_t)seg * query_seg_cap(L) : nullptr;
         uint32_t* tn = queries ? n_queries + seg * kQueryCtrStride : nullptr;
