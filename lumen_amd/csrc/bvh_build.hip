@@ -1104,8 +1104,10 @@ lt_status bvh_build(lt_context* ctx, const lt_build_opts* opts, lt_build_stats* 
         if (verdict != 0xFFFFFFFFu)
             return lt_fail(ctx, LT_ERR_HIP, "BVH8 node " + std::to_string(verdict - 1u) + " has a bad child or leaf");
         for (int k = 0; k < 3; k++) {
-            bvh.root_p[k] = root.p[k];
-            bvh.root_x[k] = std::ldexp(131072.0f, root.e[k]);
+            // non-negative fp16 bit patterns are ordered as their values; an empty slot's is 0
+            const uint16_t q = *std::max_element(root.qhi[k], root.qhi[k] + 8);
+            bvh.root_lo[k] = root.p[k];
+            bvh.root_hi[k] = root.p[k] + std::ldexp((float)__builtin_bit_cast(_Float16, q), root.e[k]);
         }
         float ms = 0.0f;
         LT_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));

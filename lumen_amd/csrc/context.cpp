@@ -45,8 +45,11 @@ SceneView make_scene_view(const lt_context* ctx) {
     v.num_lights = s.nlights;
     v.num_nodes = ctx->bvh.built ? ctx->bvh.n_nodes : 0;
     v.deep_stack = ctx->bvh.depth > (uint32_t)ltb::kLdsStack + 1u ? 1u : 0u;
-    memcpy(v.root_p, ctx->bvh.root_p, sizeof(v.root_p));
-    memcpy(v.root_x, ctx->bvh.root_x, sizeof(v.root_x));
+    for (int k = 0; k < 3; k++) {
+        v.root_lo[k] = ctx->bvh.root_lo[k];
+        v.root_hi[k] = ctx->bvh.root_hi[k];
+        v.root_x[k] = v.root_hi[k] - v.root_lo[k];
+    }
     v.refill_min = ctx->tuning.refill_min;
     v.total_light_triangle_cnt = s.total_light_triangle_cnt;
     v.dir_light_idx = s.dir_light_idx;

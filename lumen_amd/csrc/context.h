@@ -39,9 +39,9 @@ struct SceneView {
     uint32_t num_lights;
     uint32_t num_nodes;
     uint32_t deep_stack;  // 1: the tree has more levels than the LDS stack serves
-    // the root node's origin, and per axis 2^17 times its scale 2^e: bounds
-    // over every node of the tree (dev_trace.h, ray_bounds)
-    float root_p[3], root_x[3];
+    // the root node's decoded box and its extent: bounds over every node of
+    // the tree (dev_trace.h, ray_bounds)
+    float root_lo[3], root_hi[3], root_x[3];
     uint32_t refill_min;  // wavefront trace stages (lt_tuning)
     uint32_t total_light_triangle_cnt;
     int32_t dir_light_idx;
@@ -84,7 +84,7 @@ struct DeviceBVH {
     ltb::Node8* nodes = nullptr;
     ltb::TriRec* tris = nullptr;
     uint32_t n_nodes = 0, n_tris = 0, depth = 0;
-    float root_p[3] = {0, 0, 0}, root_x[3] = {0, 0, 0};  // SceneView::root_p, root_x
+    float root_lo[3] = {0, 0, 0}, root_hi[3] = {0, 0, 0};  // SceneView::root_lo, root_hi
     bool built = false;
 };
 

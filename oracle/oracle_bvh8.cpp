@@ -59,19 +59,22 @@ extern "C" void ora_bvh8_trace(const void* nodes_v, uint32_t n_nodes, const void
         uint32_t best_gid = 0xFFFFFFFFu, best_prim = 0xFFFFFFFFu, best_inst = 0xFFFFFFFFu;
         uint64_t nn = 0, nt = 0;
         bool done = false;
-        // rounding bounds of the ray over every node of the tree (from the
-        // root): E of a slab distance per axis, 2^-21 F with
-        // F = |1/d| (|p_r - o| + 2^17 2^e_r) >= 65535 |a| + |b| of any node, and
-        // the cull margin, 2^-16 F along the dominant axis kz (the error of a
+        // rounding bounds of the ray over every node of the tree, from the root's
+        // box [lo, hi], with M the larger distance of its planes from the origin:
+        // E = 2^-21 |1/d| (M + hi - lo) of a slab distance per axis, and the cull
+        // margin, 2^-16 |1/d| M along the dominant axis kz (the error of a
         // triangle's watertight t)
         float E[3] = {0, 0, 0}, margin = 0.0f;
         if (n_nodes) {
             const float adx = fabsf(d.x), ady = fabsf(d.y), adz = fabsf(d.z);
             const int kz = (adx > ady) ? (adx > adz ? 0 : 2) : (ady > adz ? 1 : 2);
             for (int k = 0; k < 3; k++) {
-                const float F = fabsf(inv[k]) * (fabsf(nodes[0].p[k] - o[k]) + ldexpf(131072.0f, nodes[0].e[k]));
-                E[k] = kSlabErr * F;
-                if (k == kz) margin = F * (1.0f / 65536.0f);
+                const Node8h& root = nodes[0];
+                const float lo = root.p[k];
+                const float hi = lo + ldexpf(f16v(*std::max_element(root.qhi[k], root.qhi[k] + 8)), root.e[k]);
+                const float a = kSlabErr * fabsf(inv[k]), M = fmaxf(fabsf(lo - o[k]), fabsf(hi - o[k]));
+                E[k] = a * (M + (hi - lo));
+                if (k == kz) margin = a * M * 32.0f;
             }
         }
         std::vector<uint32_t> stack;

@@ -48,6 +48,30 @@ def test_rays_that_cannot_hit_visit_no_node(any_hit):
     assert nc.max() <= 1 and tc.max() == 0, (nc.max(), tc.max())
 
 
+@pytest.mark.parametrize("scale", [1.0, 37.0, 2.0 ** -20])
+def test_the_surfaces_at_a_rays_ends_are_not_tested(scale):
+    """The cull margin is 2^-16 of the farthest point of the scene along the ray's
+    dominant axis (and the slab error 2^-20 of the extent): segments between two
+    walls of a box of extent 1 that keep 2^-15 from both test no triangle."""
+    from scenes import box_faces
+    tri = np.concatenate([np.array(f, np.float32) for f in box_faces((0, 0, 0), (1, 1, 1))])
+    tri *= np.float32(scale)
+    nodes, tris = host_bvh8.build(tri)
+    rng = np.random.default_rng(2)
+    n = 600
+    r = np.zeros(n, RAY_DTYPE)
+    ax, up = rng.integers(0, 3, n), rng.random(n) < 0.5
+    o, d = rng.uniform(0.3, 0.7, (n, 3)), rng.uniform(-0.2, 0.2, (n, 3))
+    i = np.arange(n)
+    gap = 2.0 ** -15
+    o[i, ax] = np.where(up, gap, 1 - gap)
+    d[i, ax] = np.where(up, 1.0, -1.0)
+    r["org"], r["dir"], r["tmin"], r["tmax"] = o * scale, d, 0.0, (1 - 2 * gap) * scale
+    occ, nc, tc = oracle.bvh8_trace(nodes, tris, r, True)
+    assert not occ.any() and nc.min() >= 1
+    assert tc.sum() == 0, tc.mean()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("any_hit", [False, True])
 def test_rays_that_cannot_hit_visit_no_node_on_the_device(gpu_ctx, any_hit):
