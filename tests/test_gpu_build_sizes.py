@@ -48,22 +48,50 @@ def test_builds_of_every_size_class(gpu_ctx, tree, collapse):
             assert np.array_equal(g.view(np.uint8), o.view(np.uint8)), (tree, collapse, k)
 
 
-def test_a_chain_too_deep_is_refused(gpu_ctx):
-    print("[gpu] too deep a chain", flush=True)
+def _nested(n):
+    """n triangles whose boxes are nested cubes, the smallest first.  A union's
+    box is the larger one's, so of all pairs only the two smallest clusters
+    prefer each other: PLOC merges one pair a round into a chain of n - 1
+    nodes, and a BVH8 node takes 7 of its triangles and the rest, whichever
+    collapse: (n - 1) / 7 levels."""
     s = DescScene()
     m = s.material(bsdf_type=1, bsdf_props=9, albedo=(0.5, 0.5, 0.5))
-    k = 2.0 ** (-0.05 * np.arange(2400))
-    base = np.array([[1, 0.2, 0], [1.2, -0.2, 0.1], [1.1, 0, 0.3]])
-    s.mesh((k[:, None, None] * base).astype(np.float32), m)
+    k = np.exp2(np.linspace(-72, 20, n))
+    base = np.array([[-1, -1, -1], [1, 1, -1], [1, -1, 1]])
+    s.mesh((k[:, None, None] * base).astype(np.float32), m, normals=np.tile(np.float32([0, 0, 1]), (n, 3, 1)))
     sc = la.Scene.__new__(la.Scene)
     sc._h = None
     sc.desc = s.build()
-    gpu_ctx.upload(sc)
-    try:
-        st = gpu_ctx.build_accel()
-        assert st.max_depth <= 192  # or a tree shallow enough
-    except la.LtError as e:
-        assert "stack bound" in str(e)
+    sc._keep = s
+    return sc
+
+
+# 1370: 193..200 levels, found after the last level; 2000: more levels than are
+# launched at all; 2600: also PLOC rounds beyond one start of their counts
+@pytest.mark.parametrize("collapse", ["sah", "greedy"])
+@pytest.mark.parametrize("n", [1370, 2000, 2600])
+def test_a_chain_too_deep_is_refused(gpu_ctx, n, collapse):
+    print(f"[gpu] too deep a chain {n} {collapse}", flush=True)
+    gpu_ctx.upload(_nested(n))
+    with pytest.raises(la.LtError, match="stack bound"):
+        gpu_ctx.build_accel(collapse=collapse)
     ok = _scene(50, 1)  # the context stays usable
     gpu_ctx.upload(ok)
     assert gpu_ctx.build_accel().num_tris == 50
+    t = ok.triangles()
+    rays = np.concatenate([random_rays(t, 300, 1), aimed_rays(t, 300, 2)])
+    g, o = gpu_ctx.trace_closest(rays), oracle.Accel(ok.desc).closest(rays, brute=True)
+    assert np.array_equal(g.view(np.uint8), o.view(np.uint8))
+
+
+def test_the_deepest_chain_is_traced(gpu_ctx):
+    print("[gpu] deepest chain", flush=True)
+    sc = _nested(1340)
+    gpu_ctx.upload(sc)
+    st = gpu_ctx.build_accel()
+    assert 185 <= st.max_depth <= 192, st.max_depth
+    t = sc.triangles()
+    rays = np.concatenate([random_rays(t[-200:], 1000, 1), aimed_rays(t[-200:], 1000, 2), aimed_rays(t[600:], 1000, 3)])
+    g, o = gpu_ctx.trace_closest(rays), oracle.Accel(sc.desc).closest(rays, brute=True)
+    assert (g["inst"] != 0xFFFFFFFF).any()
+    assert np.array_equal(g.view(np.uint8), o.view(np.uint8))
