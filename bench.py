@@ -429,8 +429,8 @@ def main() -> int:
     ap.add_argument("--cpu-seconds", type=float, default=15.0)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--strategy", choices=["persistent", "wavefront", "megakernel"], default="persistent",
-                    help="Path execution form: persistent wavefront stages, one persistent kernel with path "
-                         "regeneration, or the per-pixel megakernel")
+                    help="Path execution form: one persistent kernel with path regeneration (megakernel runs "
+                         "the same one) or persistent wavefront stages")
     ap.add_argument("--gt-frames", type=int, default=-1,
                     help="ground-truth frames of the time-to-RMSE measurement (0 skips it; default 1024 for "
                          "path and bdpt, 128 for vcm)")
@@ -594,8 +594,7 @@ def main() -> int:
     else:
         workload = "terrain-1M+2000-boxes-1920x1080-path-d12"
         out_integrator = f"path-{args.strategy}"
-        roof = line(
-                    "k_path_regen (one launch per frame)" if args.strategy != "wavefront" else
+        roof = line("k_path_regen (one launch per frame)" if args.strategy != "wavefront" else
                     "one frame's launch sequence (trace + shade per depth)", bvh_bytes, avg_ms)
     roof["traffic"] = traffic_from_profile(workload, out_integrator)
 

@@ -252,8 +252,11 @@ typedef struct lt_build_stats {
 
 /* Replaces Integrator::create_accel -> vk::build_blas / vk::build_tlas
  * (src/RayTracer/Integrator.cpp:137-160, src/Framework/AccelerationStructure.cpp:171-315):
- * LBVH (30-bit Morton, radix sort, Karras radix tree) collapsed to a BVH8 of
- * 128-byte quantised nodes.  opts may be NULL. */
+ * a binary tree over the Morton-sorted triangles (lt_build_opts) collapsed to a
+ * BVH8 of 128-byte quantised nodes.  opts may be NULL.  The context keeps the
+ * build's workspace, about 360 B per triangle, for its next build if it is at
+ * most 512 MiB (a first build, which allocates it, takes longer), until the
+ * context is destroyed. */
 lt_status lt_accel_build(lt_context* ctx, const lt_build_opts* opts, lt_build_stats* stats);
 /* Copies the built BVH8 (128-B nodes) and its 48-B triangle records to host
  * memory (for inspection and for host traversals over the identical tree).
@@ -299,12 +302,14 @@ typedef struct lt_tuning {
                                       most what a CU holds                              */
     uint32_t refill_min;           /* raw queries and wavefront trace stages: idle lanes
                                       that trigger a refill, 1..64 (default 32)         */
-    uint32_t bdpt_blocks_per_cu;   /* BDPT and VCM persistent kernels, 128-thread
-                                      workgroups; default 0 = each kernel's resident
-                                      workgroups per CU (its register and LDS use).
+    uint32_t bdpt_blocks_per_cu;   /* BDPT, VCM and SPPM persistent kernels, 128-thread
+                                      workgroups, at most what a CU holds; default 0 =
+                                      each kernel's resident workgroups per CU (its
+                                      register and LDS use).
                                       lt_set_tuning leaves a 0 field unchanged.         */
-    uint32_t regen_min;            /* persistent Path kernel and BDPT walk: idle lanes
-                                      that trigger taking new pixels, 1..64 (default 4) */
+    uint32_t regen_min;            /* persistent Path kernel, BDPT walk, VCM light pass and
+                                      SPPM eye pass: idle lanes that trigger taking new
+                                      paths, 1..64 (default 4)                           */
     uint32_t bdpt_chunk_tiles;     /* BDPT: 8x8 pixel tiles per walk/connection pass,
                                       read when an integrator is created; default 0 =
                                       as many as fit a 4 GiB vertex store               */
@@ -482,7 +487,9 @@ lt_status lt_integrator_create(lt_context* ctx, lt_integrator_kind kind, const v
 lt_status lt_integrator_destroy(lt_integrator* it);
 /* Replaces Integrator::render + RenderGraph::run (src/RayTracer/Path.cpp:27-59):
  * renders params->spp frames starting at params->frame_num into the running
- * mean.  Asynchronous. */
+ * mean.  Asynchronous.  A Path integrator (persistent, megakernel) that renders
+ * several frames at once keeps their samples, 16 B per pixel and frame up to
+ * 512 MiB, until it is destroyed; without that memory it goes frame by frame. */
 lt_status lt_render(lt_integrator* it, const lt_frame_params* params);
 /* Ray counts and device time of the last lt_render (synchronises; with
  * counting enabled the kernels tally rays). */
@@ -530,7 +537,12 @@ typedef struct lt_adjoint_config {
     float sky_col[3];
     uint32_t reserved[8];
 } lt_adjoint_config;
-/* Requires lt_scene_upload and lt_accel_build on ctx. */
+/* Requires lt_scene_upload and lt_accel_build on ctx.  The object keeps device
+ * memory until lt_adjoint_destroy: the traversal stacks' spill (132 MiB);
+ * for 8 or more variants the rays they share, about 12 MiB per bounce up to 16
+ * bounces; for 4 or more variants whose samples outnumber the texels, the
+ * texels and their gradients once more, interleaved, up to 4 GiB.  Where the
+ * last two cannot be had it works without them. */
 lt_status lt_adjoint_create(lt_context* ctx, const lt_adjoint_config* cfg, lt_adjoint** out);
 lt_status lt_adjoint_destroy(lt_adjoint* adj);
 /* Texel grids of the two replaced textures (0 x 0 for a texture set to -1). */

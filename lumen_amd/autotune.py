@@ -35,14 +35,14 @@ TABLE = Path(__file__).resolve().parent / "tuning.json"
 
 # candidate values per lt_tuning field and workload
 SPACE = {
-    "path-persistent": {"path_blocks_per_cu": [6, 8, 10, 12, 16], "regen_min": [1, 2, 4, 8, 16, 32],
-                        "xcd_bands": [1, 2]},
-    "path-megakernel": {"path_blocks_per_cu": [4, 6, 8, 10, 12, 16]},
+    "path-persistent": {"path_blocks_per_cu": [6, 8, 10, 12, 16], "regen_min": [1, 2, 4, 8, 16, 32]},
+    # runs the persistent kernel
+    "path-megakernel": {"path_blocks_per_cu": [6, 8, 10, 12, 16], "regen_min": [1, 2, 4, 8, 16, 32]},
     "path-wavefront": {"path_blocks_per_cu": [6, 8, 10, 12, 16], "refill_min": [8, 16, 32, 48, 64],
                        "wf_sort": [1, 2]},
     "bdpt": {"bdpt_blocks_per_cu": [2, 3, 4, 6, 8], "regen_min": [1, 2, 4, 8, 16]},
-    "vcm-corrected": {"bdpt_blocks_per_cu": [2, 3, 4, 6, 8]},
-    "sppm": {"bdpt_blocks_per_cu": [2, 3, 4, 6, 8]},
+    "vcm-corrected": {"bdpt_blocks_per_cu": [2, 3, 4, 6, 8], "regen_min": [1, 2, 4, 8, 16]},
+    "sppm": {"bdpt_blocks_per_cu": [2, 3, 4, 6, 8], "regen_min": [1, 2, 4, 8, 16]},
 }
 
 # build-time sizes (preprocessor definitions of bvh_layout.h / dev_trace.h)

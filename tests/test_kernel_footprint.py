@@ -2,8 +2,8 @@
 capped with amdgpu_waves_per_eu (CPU only: read from the compiler's
 kernel-resource-usage remarks that lumen_amd/build.py records).
 
-Three of these kernels once produced wrong images at tighter caps (the Path
-megakernel at 5 waves per SIMD, the VCM light pass and the adjoint at 4), a
+Three kernels once produced wrong images at tighter caps (an earlier Path
+kernel at 5 waves per SIMD, the VCM light pass and the adjoint at 4), a
 result that depended on how the compiler allocated registers and spilled.
 The shipped caps and the current footprints are the ones the GPU replay
 tests validate, so any change of a capped kernel's registers, scratch or
@@ -49,6 +49,7 @@ def test_trace_kernels_fit_the_lds_budget(resources):
     """Every traversal kernel holds kLdsWords (32) words per thread of
     128-thread workgroups in LDS: 16 KiB per workgroup, so that ten
     workgroups fit the 160 KiB of a CU."""
-    for name, v in resources.items():
-        if any(t in name for t in ("k_path_regen", "k_path_mega", "k_bdpt_walk", "k_vcm_light", "k_sppm_eye")):
-            assert v["lds_bytes"] == 16384, name
+    kernels = ("k_path_regen", "k_bdpt_walk", "k_vcm_light", "k_sppm_eye")
+    for t in kernels:
+        found = [v["lds_bytes"] for name, v in resources.items() if t in name]
+        assert found and all(b == 16384 for b in found), (t, found)
