@@ -78,9 +78,9 @@ extern "C" void ora_bvh8_trace(const void* nodes_v, uint32_t n_nodes, const void
             }
         }
         std::vector<uint32_t> stack;
-        // a ray with a NaN, or an empty interval, hits nothing and visits no node
+        // a ray with a NaN in its origin or direction hits nothing and visits no node
         const float Es = E[0] + E[1] + E[2];
-        if (n_nodes && Es == Es && tmin - margin <= tmax + margin) stack.push_back(0);
+        if (n_nodes && Es == Es) stack.push_back(0);
         while (!stack.empty() && !done) {
             const Node8h& nd = nodes[stack.back()];
             stack.pop_back();
