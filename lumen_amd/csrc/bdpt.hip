@@ -1,10 +1,11 @@
 // bdpt.hip — the BDPT integrator on gfx950.
 //
-// A frame runs over chunks of 8x8 pixel tiles with two persistent kernels per
-// chunk: the walk kernel traces each pixel's light and camera subpaths
-// (bdpt_commons.glsl:13-270) into a structure-of-arrays vertex buffer, then
-// the connection kernel evaluates every (s, t) strategy of bdpt.rgen:53-76.
-// Splitting the two keeps each kernel's register footprint, and so its
+// A frame runs over chunks of 8x8 pixel tiles with three kernels per chunk: the
+// walk kernel (persistent) traces each pixel's light and camera subpaths
+// (bdpt_commons.glsl:13-270) into a structure-of-arrays vertex buffer, the
+// prefix kernel adds each vertex's MIS prefix, a thread per subpath, and the
+// connection kernel (persistent) evaluates every (s, t) strategy of
+// bdpt.rgen:53-76.  Splitting walk and connection keeps each kernel's register footprint, and so its
 // occupancy, to its own phase.  Light-tracing strategies (t = 1) add their
 // splat to the target pixel with float atomics; a last kernel adds each
 // pixel's splats to its camera-side estimate and applies the NaN guard and

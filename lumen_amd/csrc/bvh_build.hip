@@ -24,6 +24,8 @@
 // counts, fences and atomics on shared lines.  250k triangles: 12.2 ms with a
 // launch and a host look per round and level, a pass each for counts, ranges
 // and tables and a host check of the nodes; 1.7 ms now (1M: 29.9 and 2.5 ms).
+// These are repeated builds: a context's first one also allocates the
+// workspace (1M: 6.5 ms).
 #include <hip/hip_runtime.h>
 
 #include <rocprim/device/device_radix_sort.hpp>

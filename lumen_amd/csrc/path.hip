@@ -1,8 +1,10 @@
 // path.hip — the Path integrator on gfx950 (persistent form).
 //
-// One thread per pixel, persistent waves pulling 8x8 pixel tiles, all frames
-// of a launch accumulated in registers with the reference's per-frame running
-// mean (path.rgen:106-112) so the result equals frame-by-frame launches.
+// Persistent lanes with path regeneration over the samples of a launch's
+// frames, dealt out in 8x8 pixel tiles (k_path_regen).  The samples of several
+// frames go to a buffer that k_path_mean folds in frame order into the
+// reference's running mean (path.rgen:106-112), so the result equals
+// frame-by-frame launches; a single frame's go straight into the mean.
 // Per-sample logic: src/shaders/integrators/path/path.rgen:26-104 and
 // src/shaders/integrators/pt_commons.glsl:3-47.
 #include <hip/hip_runtime.h>

@@ -1,5 +1,6 @@
 // trace.hip — raw closest-hit / any-hit kernels behind lt_trace_closest,
-// lt_trace_any and lt_trace_count (persistent waves pulling 64 rays at a time).
+// lt_trace_any and lt_trace_count: persistent waves over dealt tiles of 64 rays,
+// a lane taking the next ray when enough lanes' rays have ended (trace_stream).
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 

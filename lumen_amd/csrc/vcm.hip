@@ -19,7 +19,8 @@
 //                 mean; the corrected one appends a merge query per
 //                 non-specular vertex and leaves the colour in fcol;
 //   k_vcm_merge   (corrected) one wave per merge query over the photons of
-//                 all its cells, sums added to fcol;
+//                 all its cells, sums added to fcol; launched a second time
+//                 for the parts of the queries that have many photons;
 //   k_vcm_resolve (corrected) fcol plus the splats into the running mean.
 // The light, eye and merge kernels are persistent.
 #include <hip/hip_runtime.h>
