@@ -440,7 +440,7 @@ def main() -> int:
     if args.stream_copy:
         return stream_copy(args.stream_copy)
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
-        print("bench.py measures one GPU only: this build has no multi-GPU path (each GPU box here has one GPU); "
+        print("bench.py measures one GPU only: this build has no multi-GPU path; "
               "run with --gpus 1", file=sys.stderr)
         return 2
 
